@@ -111,6 +111,17 @@ hipError_t qe_attn_prefill(const void* q, const void* kc, const void* vc, const 
                            const void* qg, long ldp, void* out, long ldo, int T, int Hq, int Hkv,
                            int max_len, float scale, hipStream_t stream);
 
+/* qe_attn_prefill with a caller's workspace, which lets a chunk that does not fill the CUs split
+ * the cache over more of them: ws of at least qe_attn_prefill_ws_size() bytes, 16-byte aligned,
+ * contents undefined before and after; calls that may overlap need one each. The size is 0 where no
+ * position in the cache would make splitting pay. A null ws, or fewer bytes, runs unsplit (as
+ * qe_attn_prefill does): the same values up to rounding. */
+size_t qe_attn_prefill_ws_size(int T, int Hq, int Hkv, int max_len);
+hipError_t qe_attn_prefill_ws(const void* q, const void* kc, const void* vc, const int* pos,
+                              const void* qg, long ldp, void* out, long ldo, int T, int Hq, int Hkv,
+                              int max_len, float scale, void* ws, size_t ws_bytes,
+                              hipStream_t stream);
+
 /* Number of cache positions per split-KV slice for a row attending L positions with NS partial
  * slots: ceil(L/NS) rounded up to a multiple of 32 (at least 32); row t's partial s covers
  * positions [s*size, (s+1)*size) of [0, L). The reference cuts ceil(L/NS) (csrc/attn.cu:78-80);
@@ -148,6 +159,10 @@ hipError_t qe_attn_prefill_fp8(const void* q, const void* kc8, const void* vc8, 
                                const void* qg, long ldp, void* out, long ldo, int T, int Hq,
                                int Hkv, int max_len, float scale, float k_scale, float v_scale,
                                hipStream_t stream);
+hipError_t qe_attn_prefill_fp8_ws(const void* q, const void* kc8, const void* vc8, const int* pos,
+                                  const void* qg, long ldp, void* out, long ldo, int T, int Hq,
+                                  int Hkv, int max_len, float scale, float k_scale, float v_scale,
+                                  void* ws, size_t ws_bytes, hipStream_t stream);
 
 /* First half of qe_attn_decode_fp8 (the partials are not yet multiplied by v_scale). */
 hipError_t qe_attn_decode_fp8_partials(const void* q, const void* kc8, const void* vc8,

@@ -19,6 +19,7 @@ _P = ctypes.c_void_p
 _I = ctypes.c_int
 _L = ctypes.c_long
 _F = ctypes.c_float
+_Z = ctypes.c_size_t
 
 SIGNATURES = {
     "qe_attn_prep": (_I, [_P, _P, _P, _L, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _F, _P]),
@@ -27,6 +28,10 @@ SIGNATURES = {
     "qe_attn_decode_noalloc": (_I, [_P, _P, _P, _P, _P, _L, _P, _L, _I, _I, _I, _I, _I, _F, _P]),
     "qe_attn_decode_combine": (_I, [_P, _P, _P, _P, _L, _P, _L, _I, _I, _I, _I, _P]),
     "qe_attn_prefill": (_I, [_P, _P, _P, _P, _P, _L, _P, _L, _I, _I, _I, _I, _F, _P]),
+    "qe_attn_prefill_ws": (_I, [_P, _P, _P, _P, _P, _L, _P, _L, _I, _I, _I, _I, _F, _P, _Z, _P]),
+    "qe_attn_prefill_fp8_ws": (_I, [_P, _P, _P, _P, _P, _L, _P, _L, _I, _I, _I, _I, _F, _F, _F, _P,
+                                    _Z, _P]),
+    "qe_attn_prefill_ws_size": (_Z, [_I, _I, _I, _I]),
     "qe_attn_prefill_fp8": (_I, [_P, _P, _P, _P, _P, _L, _P, _L, _I, _I, _I, _I, _F, _F, _F, _P]),
     "qe_attn_prep_decode": (_I, [_P, _P, _P, _L, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _L, _I, _I,
                                  _I, _I, _I, _I, _F, _F, _P]),

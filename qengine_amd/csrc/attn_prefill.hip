@@ -4,14 +4,17 @@
 // python/qengine/reference.py:263-272). The reference has no prefill kernel: it feeds prompts
 // through its n <= 8 row decode path (engine.py:542-573).
 //
-// Design (compute-bound, MFMA):
-//  * Workgroup = 128 consecutive query rows of one q head: 8 waves x 16 rows (one 16-column MFMA
-//    tile per wave, two waves per SIMD). Workgroups are dispatched heaviest (longest attended prefix) first
-//    over the whole grid, which balances the causal triangle across the CUs, and the workgroups of
-//    one KV head are placed on the same XCDs (one L2 per XCD).
-//  * K/V tiles of 32 positions are streamed into a 4-stage LDS ring by LDS DMA (each wave fetches
-//    4 rows of K and of V, three tiles ahead, one barrier per tile) and shared by the 8 waves. K
-//    and V are XOR-swizzled for conflict-free operand reads (rocprofv3: zero LDS bank conflicts).
+// Two kernels; launch_prefill chooses:
+//  * attn_prefill_wide_kernel (attn_prefill_wide.hip): any shape.
+//  * attn_prefill_bal_kernel (here): GQA 6 where its 16-row blocks of all heads fill one round of the
+//    CUs (T about 2,048 at 24 / 4 heads). 12 waves (three per SIMD) of one KV head own three quads of
+//    (16-row block, q head) units, four units of one length per quad, one unit of each quad per
+//    SIMD; the quads of a workgroup mix lengths so that every workgroup carries about the same work.
+//
+// The balanced kernel (compute-bound, MFMA):
+//  * K/V tiles of 32 positions are streamed into a 4-stage LDS ring by LDS DMA (each of the first 8
+//    waves fetches 4 rows of K and of V, one barrier per tile) and shared by the 12 waves. K and V
+//    are XOR-swizzled for conflict-free operand reads (rocprofv3: zero LDS bank conflicts).
 //  * The V^T operands of PV come straight from LDS through gfx950's transposing read
 //    (ds_read_b64_tr_b16), so no VALU permutes assemble them.
 //  * Per tile and wave: S^T = K Q^T (16 MFMA 16x16x32), online softmax per column in the log2
@@ -23,31 +26,20 @@
 //    tiles run as two loops, and the hi/lo choice is made once per wave, so the accumulators stay
 //    in one register class across iterations.
 //  * Epilogue: O / l rounded to bf16, times bf16(sigmoid(gate)), 8-byte stores.
-//  * At GQA 6 (bf16 and fp8 caches), attn_prefill_bal_kernel runs the same per-wave code in a
-//    layout that balances the causal triangle: 12 waves (three per SIMD) of one KV head own
-//    three quads of (16-row block, q head) units, four units of one length per quad, one unit of
-//    each quad per SIMD; the quads of a workgroup mix lengths so that every workgroup carries
-//    about the same work, and the grid is one round of workgroups (config 5: 256). Same bits as
-//    the 8-wave kernel. Its first form (blocks j and nb-1-j, one q head per wave): 222 -> 212 us
-//    at config 5 (same-box A/B); on the fp8 cache it replaced the 8-wave kernel: 290 -> 243 us.
 //  * The file is compiled with LLVM's max-ILP machine scheduler. Under the default
 //    (occupancy-first) scheduler the tile loop kept one LDS operand read in flight and waited
 //    for it before every MFMA; max-ILP interleaves the two S^T accumulation chains and keeps two
 //    or more reads in flight in the same 168 registers. Same bits; config 5, same-box A/B against
 //    the default scheduler: 207.8 -> 189.3 us (bf16 cache), 243.7 -> 224.7 us (fp8 cache).
+#include "attn_prefill.hpp"
 #include "attn_tile.hpp"
 #include "qe_attn.h"
 
 namespace qe {
 namespace prefill {
 
-// Two waves per SIMD: one wave's softmax (VALU) overlaps the other's MFMAs. With 16 rows per
-// wave the tile loop fits 218 VGPRs. (Measured on MI355X at config 5: 4 waves x 32 rows, one wave
-// per SIMD, ran 328 us; 8 waves x 16 rows runs 271 us.)
-constexpr int WAVES = 8;
-constexpr int ROWS_PER_WAVE = 16;               // one 16-column MFMA tile per wave
-constexpr int NT = ROWS_PER_WAVE / 16;
-constexpr int BQ = WAVES * ROWS_PER_WAVE;       // 128 query rows per workgroup
+constexpr int WAVES = 8;                        // waves that load the ring
+constexpr int NT = 1;                           // 16-column MFMA tiles per wave
 using tile::BN;                                 // cache positions per step
 using tile::ROW_CHUNKS;
 // Rows attending at least this many positions use one bf16 term for P (error ~2^-9/sqrt(N) of
@@ -56,11 +48,10 @@ constexpr int SPLIT_BELOW = 512;
 constexpr int TILE_U4 = BN * ROW_CHUNKS;        // 16-byte slots per K (or V) tile: 1024
 constexpr int STAGE_U4 = 2 * TILE_U4;           // K tile then V tile (32 KB)
 constexpr int STAGES = 4;                       // LDS ring of tiles
-constexpr int AHEAD = STAGES - 1;               // tiles in flight beyond the one computed
 constexpr int LOAD_ROWS = BN / WAVES;            // K and V rows each wave fetches per tile
 constexpr int LOAD_INSTR = LOAD_ROWS / 2;        // two 512-byte rows per LDS-DMA instruction
 constexpr int LOADS_PER_TILE = 2 * LOAD_INSTR;   // K then V
-static_assert(LOAD_ROWS % 2 == 0 && LOADS_PER_TILE * AHEAD < 64, "tile split over the waves");
+static_assert(LOAD_ROWS % 2 == 0, "tile split over the waves");
 constexpr int PF_CPOL = 0;                      // cached loads: every row block re-reads its KV head
 constexpr int XCDS = 8;                         // MI355X: 8 XCDs, each with its own L2
 // Operand reads kept ahead of the MFMAs in a tile's S^T and O^T steps (tile::qk_tile / pv_tile_tr
@@ -93,34 +84,6 @@ struct WaveState {
   float m[NT], l[NT];
   f32x4_t acc[NT][16];  // acc[ct][i][k] = O^T[16i + 4 g4 + k][column ct*16 + c] (tile::pv_tile_tr)
 };
-
-// Tiles [j0, j1) of the ring with one branch-free body (SPLIT and MASK fixed).
-template <bool SPLIT, bool MASK>
-__device__ __forceinline__ void run_tiles(int j0, int j1, int Lwave, u32x4_t* lds,
-                                          __amdgpu_buffer_rsrc_t krs, __amdgpu_buffer_rsrc_t vrs,
-                                          int w, int lane, int c, int g4,
-                                          const bf16x8_t (&qb)[NT][8], const int (&Lcol)[NT],
-                                          float scale_log2, WaveState& st) {
-  for (int j = j0; j < j1; ++j) {
-    const u32x4_t* kt = lds + (j % STAGES) * STAGE_U4;
-    const u32x4_t* vt = kt + TILE_U4;
-    const int p0 = j * BN;
-    vmcnt_wait<LOADS_PER_TILE * (AHEAD - 1)>();  // this wave's loads of tile j are done
-    __syncthreads();                // ... and every wave's; tile j-1's stage is free
-    // the arithmetic on tile j first, then the loads of tile j + AHEAD: GQA 4 / 8 shapes of
-    // config 5 231.3 / 145.0 -> 225.6 / 140.0 us against issuing the loads first (same bits)
-    if (p0 < Lwave) {  // tiles past this wave's rows contribute nothing
-      f32x4_t sacc[NT][2];
-      tile::qk_tile<NT, NT == 1, SG_LEAD>(kt, qb, c, g4, sacc);
-      u32x4_t pb_hi[NT], pb_lo[NT];
-      tile::softmax_tile<NT, MASK, SPLIT>(sacc, p0, Lcol, scale_log2, g4, st.m, st.l, st.acc,
-                                          pb_hi, pb_lo);
-      tile::pv_tile_tr<NT, SPLIT, NT == 1, SG_LEAD>(vt, lane, g4, pb_hi, pb_lo, st.acc);
-    }
-    if (w < WAVES)  // the first WAVES waves load the ring
-      issue_tile(lds + ((j + AHEAD) % STAGES) * STAGE_U4, krs, vrs, p0 + AHEAD * BN, w, lane);
-  }
-}
 
 // ---- fp8 KV cache (E4M3FN codes, 256-byte rows). Tiles arrive in a STAGES-deep fp8 ring by LDS
 // DMA (each wave fetches its 4 rows of K and of V: one 1 KB instruction each). One tile before
@@ -161,178 +124,8 @@ __device__ __forceinline__ void convert_tile8(const u32x4_t* stage, u32x4_t* bf)
   bf[TILE_U4 + r * ROW_CHUNKS + ((q + 1 - p) ^ tile::v_swz(r))] = fp8x8_to_bf16x8(vb);
 }
 
-// run_tiles for the fp8 cache, converting one tile ahead: iteration j computes tile j from bf16
-// pair j % 2, then converts tile j + 1 into pair (j + 1) % 2 (whose previous tile, j - 1, every
-// wave finished before this iteration's barrier), so one barrier per tile orders both. Tile j's
-// fp8 stage is free once converted, so iteration j refills it with tile j + STAGES and loads
-// still run STAGES - 1 iterations ahead of their conversion. Same bits throughout; config 5
-// shapes at GQA 4 / 8: converting tile j between two barriers, then computing it, 277.8 / 178.1
-// us; one barrier, converting before the arithmetic 264.5 / 169.3 (266.3 / 169.5 on another
-// box); after it 257.9 / 163.3.
-template <bool SPLIT, bool MASK>
-__device__ __forceinline__ void run_tiles8(int j0, int j1, int Lwave, u32x4_t* lds,
-                                           __amdgpu_buffer_rsrc_t krs, __amdgpu_buffer_rsrc_t vrs,
-                                           int w, int lane, int c, int g4,
-                                           const bf16x8_t (&qb)[NT][8], const int (&Lcol)[NT],
-                                           float scale_log2, WaveState& st) {
-  u32x4_t* bfp = lds + STAGES * STAGE8_U4;
-  for (int j = j0; j < j1; ++j) {
-    const int p0 = j * BN;
-    vmcnt_wait<LOADS_PER_TILE8 * (STAGES - 2)>();  // this wave's loads of tile j + 1 are done
-    // ... and every wave's; bf16 tile j is complete, tile j's fp8 stage and pair (j + 1) % 2 free
-    __syncthreads();
-    issue_tile8(lds + (j % STAGES) * STAGE8_U4, krs, vrs, p0 + STAGES * BN, w, lane);
-    if (p0 < Lwave) {
-      const u32x4_t* bf = bfp + (j & 1) * STAGE_U4;
-      f32x4_t sacc[NT][2];
-      tile::qk_tile<NT, NT == 1, SG_LEAD>(bf, qb, c, g4, sacc);
-      u32x4_t pb_hi[NT], pb_lo[NT];
-      tile::softmax_tile<NT, MASK, SPLIT>(sacc, p0, Lcol, scale_log2, g4, st.m, st.l, st.acc, pb_hi,
-                                          pb_lo);
-      tile::pv_tile_tr<NT, SPLIT, NT == 1, SG_LEAD>(bf + TILE_U4, lane, g4, pb_hi, pb_lo, st.acc);
-    }
-    convert_tile8(lds + ((j + 1) % STAGES) * STAGE8_U4, bfp + ((j + 1) & 1) * STAGE_U4);
-  }
-}
-
-// KV8: kc/vc hold fp8 codes (one byte per value); v_scale multiplies O / l before its bf16
-// rounding (exactly 1 for the bf16 cache).
-template <bool KV8>
-__global__ void __launch_bounds__(WAVES * WAVE)
-attn_prefill_kernel(const __bf16* __restrict__ q, const void* __restrict__ kc,
-                    const void* __restrict__ vc, const int* __restrict__ pos_ptr,
-                    const __bf16* __restrict__ qg, long ldp, __bf16* __restrict__ out, long ldo,
-                    int T, int Hq, int Hkv, int max_len, float scale_log2, float v_scale,
-                    int xcd_split) {
-  const int grp = Hq / Hkv;
-  const int nblk = (T + BQ - 1) / BQ;
-  int blk, h;
-  if (xcd_split > 0) {
-    // Workgroups are dispatched round-robin over the XCDs (linear id L -> XCD L % 8). The
-    // xcd_split XCDs 8g/Hkv .. serve KV head g only, taking turns along its work list (row block
-    // heaviest first, then q head), so the workgroups that read one KV head's cache share an L2
-    // and every XCD gets the same mix of heavy and light blocks.
-    const int L = blockIdx.x, x = L % XCDS;
-    const int i = (L / XCDS) * xcd_split + x % xcd_split;  // index in KV head g's work list
-    blk = nblk - 1 - i / grp;
-    h = (x / xcd_split) * grp + i % grp;
-  } else {
-    blk = nblk - 1 - (int)(blockIdx.x / Hq);  // heaviest (latest) row block first
-    h = blockIdx.x % Hq;
-  }
-  const int g = h / grp;
-  const int lane = threadIdx.x & (WAVE - 1), w = threadIdx.x / WAVE;
-  const int c = lane & 15, g4 = lane >> 4;
-  const int pos0 = pos_ptr[0];
-
-  __shared__ __attribute__((aligned(256))) u32x4_t lds[STAGES * STAGE_U4];  // 128 KB
-
-  // Q^T as the MFMA B operand: column ct*16 + c is chunk row r = blk*128 + 32w + 16ct + c.
-  bf16x8_t qb[NT][8];
-  int Lcol[NT];
-#pragma unroll
-  for (int ct = 0; ct < NT; ++ct) {
-    const int r = blk * BQ + w * ROWS_PER_WAVE + ct * 16 + c;
-    if (r < T) {
-      Lcol[ct] = min(pos0 + r + 1, max_len);
-      const u32x4_t* src = reinterpret_cast<const u32x4_t*>(q + (size_t)r * Hq * HD + (size_t)h * HD);
-#pragma unroll
-      for (int ks = 0; ks < 8; ++ks) qb[ct][ks] = as_bf16x8(src[4 * ks + g4]);
-    } else {
-      Lcol[ct] = 0;
-#pragma unroll
-      for (int ks = 0; ks < 8; ++ks) qb[ct][ks] = as_bf16x8(u32x4_t{0u, 0u, 0u, 0u});
-    }
-  }
-  // Longest attended prefix of this workgroup's rows and of this wave's rows; shortest among the
-  // wave's real rows (its first row): tiles reaching past it need the per-position mask, and it
-  // decides whether P is split.
-  const int last_row = min(blk * BQ + BQ, T) - 1;
-  const int Lwg = min(pos0 + last_row + 1, max_len);
-  const int r_first = blk * BQ + w * ROWS_PER_WAVE;
-  const int Lwave = min(pos0 + min(r_first + ROWS_PER_WAVE, T), max_len);
-  const int Lmin = min(pos0 + r_first + 1, max_len);
-  const int ntiles = Lwg > 0 ? (Lwg + BN - 1) / BN : 0;
-  const bool split = Lmin < SPLIT_BELOW;
-
-  constexpr int ELEM = KV8 ? 1 : 2;  // bytes per cache value
-  const size_t head_off = (size_t)g * max_len * HD * ELEM;  // bytes
-  const uint32_t bytes = (uint32_t)max(Lwg, 0) * (uint32_t)(HD * ELEM);  // past Lwg reads 0
-  const __amdgpu_buffer_rsrc_t krs = make_rsrc(static_cast<const char*>(kc) + head_off, bytes);
-  const __amdgpu_buffer_rsrc_t vrs = make_rsrc(static_cast<const char*>(vc) + head_off, bytes);
-
-  WaveState st;
-#pragma unroll
-  for (int ct = 0; ct < NT; ++ct) {
-    st.m[ct] = -INFINITY;
-    st.l[ct] = 0.f;
-#pragma unroll
-    for (int a = 0; a < 16; ++a) st.acc[ct][a] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  }
-
-  // Ring of STAGES tiles, AHEAD in flight. One barrier per tile: after the barrier of tile j every
-  // wave has finished tile j-1, whose stage is the one refilled with tile j+AHEAD.
-  // Tiles below jm need no per-position mask (every real row of the wave attends them fully).
-  const int jm = min(ntiles, max(Lmin, 0) / BN);
-  if constexpr (KV8) {
-#pragma unroll
-    for (int a = 0; a < STAGES; ++a) issue_tile8(lds + a * STAGE8_U4, krs, vrs, a * BN, w, lane);
-    vmcnt_wait<LOADS_PER_TILE8 * (STAGES - 1)>();  // this wave's loads of tile 0 are done
-    __syncthreads();                                // ... and every wave's
-    convert_tile8(lds, lds + STAGES * STAGE8_U4);  // the loop converts one tile ahead
-    if (split) {
-      run_tiles8<true, false>(0, jm, Lwave, lds, krs, vrs, w, lane, c, g4, qb, Lcol, scale_log2, st);
-      run_tiles8<true, true>(jm, ntiles, Lwave, lds, krs, vrs, w, lane, c, g4, qb, Lcol, scale_log2, st);
-    } else {
-      run_tiles8<false, false>(0, jm, Lwave, lds, krs, vrs, w, lane, c, g4, qb, Lcol, scale_log2, st);
-      run_tiles8<false, true>(jm, ntiles, Lwave, lds, krs, vrs, w, lane, c, g4, qb, Lcol, scale_log2, st);
-    }
-  } else {
-#pragma unroll
-  for (int a = 0; a < AHEAD; ++a) issue_tile(lds + a * STAGE_U4, krs, vrs, a * BN, w, lane);
-  if (split) {
-    run_tiles<true, false>(0, jm, Lwave, lds, krs, vrs, w, lane, c, g4, qb, Lcol, scale_log2, st);
-    run_tiles<true, true>(jm, ntiles, Lwave, lds, krs, vrs, w, lane, c, g4, qb, Lcol, scale_log2, st);
-  } else {
-    run_tiles<false, false>(0, jm, Lwave, lds, krs, vrs, w, lane, c, g4, qb, Lcol, scale_log2, st);
-    run_tiles<false, true>(jm, ntiles, Lwave, lds, krs, vrs, w, lane, c, g4, qb, Lcol, scale_log2, st);
-  }
-  }
-  vmcnt_wait<0>();  // no LDS DMA may still target this workgroup's LDS when it exits
-
-  // Epilogue: rows of this wave, 4 consecutive dims 16i + 4 g4 .. +3 per (ct, i) per lane.
-#pragma unroll
-  for (int ct = 0; ct < NT; ++ct) {
-    const float L = group4_sum(st.l[ct]);
-    const int r = blk * BQ + w * ROWS_PER_WAVE + ct * 16 + c;
-    if (r >= T) continue;
-    const __bf16* gp = qg + (size_t)r * ldp + (size_t)h * 2 * HD + HD;
-    __bf16* op = out + (size_t)r * ldo + (size_t)h * HD;
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const int d0 = 16 * i + 4 * g4;
-      const u32x2_t gb = *reinterpret_cast<const u32x2_t*>(gp + d0);
-      u32x2_t ob;
-#pragma unroll
-      for (int k = 0; k < 2; ++k) {
-        const float o0 = round_bf16((st.acc[ct][i][2 * k] / L) * v_scale);
-        const float o1 = round_bf16((st.acc[ct][i][2 * k + 1] / L) * v_scale);
-        const float s0 = round_bf16(sigmoid_f32(lo_bf16(gb[k])));
-        const float s1 = round_bf16(sigmoid_f32(hi_bf16(gb[k])));
-        ob[k] = pack_bf16x2(o0 * s0, o1 * s1);
-      }
-      *reinterpret_cast<u32x2_t*>(op + d0) = ob;
-    }
-  }
-}
-
-// Balanced layout for GQA 6: a workgroup of 12 waves (three per SIMD) owns KV head g and the pair
-// of 16-row blocks j and nb-1-j (light and heavy: their attended lengths add up to about the same
-// for every j) for all 6 q heads of the group. Waves 0-5 take block j of heads 0-5, waves 6-11
-// block nb-1-j. Every workgroup then carries about the same work, and Hkv * nb/2 of them fill the
-// CUs in one round (256 at config 5). The first 8 waves load the K/V ring as in the 8-wave kernel,
-// 2 tiles ahead in the 4-stage ring (config 5 under the max-ILP scheduler: 189.3 us against 190.5
-// with 3 ahead).
+// 12 waves, three per SIMD; the first 8 load the K/V ring 2 tiles ahead (config 5: 189.3 us against
+// 190.5 with 3 ahead).
 constexpr int BAL_WAVES = 12;
 constexpr int BAL_GRP = 6;
 constexpr int BAL_AHEAD = 2;
@@ -386,8 +179,8 @@ __device__ __forceinline__ void run_tiles_bal(int j0, int j1, int Lwave, u32x4_t
   }
 }
 
-// run_tiles_bal on the fp8 cache: the fp8 ring and the double-buffered bf16 pair of
-// run_tiles8, loaded and converted by the first 8 waves (LOAD; 512 threads, one 16-byte chunk of
+// run_tiles_bal on the fp8 cache: an fp8 ring and a double-buffered bf16 pair, loaded and
+// converted by the first 8 waves (LOAD; 512 threads, one 16-byte chunk of
 // K and of V each), one tile ahead: iteration j computes tile j from pair j % 2, then the loading
 // waves convert tile j + 1 into pair (j + 1) % 2, so one barrier per tile serves both (the tile
 // converted before the barrier of iteration j is tile j). Tile j's fp8 stage is free once it has
@@ -583,57 +376,89 @@ attn_prefill_bal_kernel(const __bf16* __restrict__ q, const void* __restrict__ k
 
 using namespace qe;
 
+// The balanced kernel's grid, if it takes the call: GQA 6 and between 96% and all of the CUs in one
+// round of workgroups. Measured at 24 / 4 heads, us per call (one process, in turn), balanced
+// against wide: 2,048 rows on 0 / 2,048 / 12,000 positions 73 / 158 / 573 against 70 / 166 / 594 (bf16
+// cache), 78 / 166 / 595 against 76 / 183 / 636 (fp8); 1,970 rows on 2,048 154 against 161. With more
+// rows (a second round) or fewer (idle CUs) the wide kernel wins: 3,000 rows on 1,000 245 against
+// 191, 1,500 on 1,000 92 against 80.
+static int balanced_grid(int T, int Hq, int Hkv) {
+  if (Hq != prefill::BAL_GRP * Hkv) return 0;
+  const long wgs = ((T + 15) / 16 + 1) / 2 * (long)Hkv;
+  const int cus = compute_units();
+  return wgs <= cus && wgs * 25 >= cus * 24L ? (int)wgs : 0;
+}
+
 static hipError_t launch_prefill(const void* q, const void* kc, const void* vc, const int* pos,
                                  const void* qg, long ldp, void* out, long ldo, int T, int Hq,
                                  int Hkv, int max_len, float scale, bool kv8, float k_scale,
-                                 float v_scale, hipStream_t stream) {
+                                 float v_scale, void* ws, size_t ws_bytes, hipStream_t stream) {
   auto a16 = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
   if (T < 1 || Hq < 1 || Hkv < 1 || Hq % Hkv != 0 || max_len < 1 || !pos ||
-      (long)((T + prefill::BQ - 1) / prefill::BQ) * Hq > 0x7fffffffL)
+      !prefill_wide_valid(T, Hq, Hkv))
     return hipErrorInvalidValue;
-  if (!a16(q) || !a16(kc) || !a16(vc) || !a16(qg) || !a16(out) || ldp % 8 != 0 || ldo % 8 != 0)
+  if (!a16(q) || !a16(kc) || !a16(vc) || !a16(qg) || !a16(out) || !a16(ws) || ldp % 8 != 0 ||
+      ldo % 8 != 0)
     return hipErrorInvalidValue;
   // byte offsets of the tiles loaded past the last attended row fit the 32-bit buffer range
-  if ((unsigned long long)(max_len + (prefill::AHEAD + 2) * prefill::BN) * HD * 2 >= (1ull << 32))
+  if ((unsigned long long)(max_len + 5 * tile::BN) * HD * 2 >= (1ull << 32))
     return hipErrorInvalidValue;
-  const int nblk = (T + prefill::BQ - 1) / prefill::BQ;
-  // KV-head-per-XCD placement when the heads divide the XCDs evenly and every XCD of a head gets
-  // the same number of workgroups; otherwise plain heaviest-first order.
-  const int per_head = prefill::XCDS % Hkv == 0 ? prefill::XCDS / Hkv : 0;
-  const int xcd_split =
-      per_head > 0 && (nblk * (Hq / Hkv)) % per_head == 0 ? per_head : 0;
-  const float scale_log2 = scale * 1.4426950408889634f * k_scale;
-  const dim3 grid(nblk * Hq), block(prefill::WAVES * WAVE);
-  const auto* Q = static_cast<const __bf16*>(q);
-  const auto* QG = static_cast<const __bf16*>(qg);
-  auto* O = static_cast<__bf16*>(out);
-  if (Hq == prefill::BAL_GRP * Hkv) {  // balanced 12-wave layout (GQA 6)
-    const int nb = (T + 15) / 16, npairs = (nb + 1) / 2;
-    const int xs = per_head > 0 && npairs % per_head == 0 ? per_head : 0;
-    const dim3 bgrid(npairs * Hkv), bblock(prefill::BAL_WAVES * WAVE);
+  if (const int grid = balanced_grid(T, Hq, Hkv)) {
+    // KV-head-per-XCD placement when the heads divide the XCDs evenly and every XCD of a head gets
+    // the same number of workgroups
+    const int per_head = prefill::XCDS % Hkv == 0 ? prefill::XCDS / Hkv : 0;
+    const int xs = per_head > 0 && grid / Hkv % per_head == 0 ? per_head : 0;
+    const float scale_log2 = scale * 1.4426950408889634f * k_scale;
+    const auto* Q = static_cast<const __bf16*>(q);
+    const auto* QG = static_cast<const __bf16*>(qg);
+    auto* O = static_cast<__bf16*>(out);
+    const dim3 block(prefill::BAL_WAVES * WAVE);
     if (kv8)
-      prefill::attn_prefill_bal_kernel<true><<<bgrid, bblock, 0, stream>>>(
+      prefill::attn_prefill_bal_kernel<true><<<grid, block, 0, stream>>>(
           Q, kc, vc, pos, QG, ldp, O, ldo, T, Hq, Hkv, max_len, scale_log2, v_scale, xs);
     else
-      prefill::attn_prefill_bal_kernel<false><<<bgrid, bblock, 0, stream>>>(
+      prefill::attn_prefill_bal_kernel<false><<<grid, block, 0, stream>>>(
           Q, kc, vc, pos, QG, ldp, O, ldo, T, Hq, Hkv, max_len, scale_log2, 1.f, xs);
     return hipGetLastError();
   }
-  if (kv8)
-    prefill::attn_prefill_kernel<true><<<grid, block, 0, stream>>>(
-        Q, kc, vc, pos, QG, ldp, O, ldo, T, Hq, Hkv, max_len, scale_log2, v_scale, xcd_split);
-  else
-    prefill::attn_prefill_kernel<false><<<grid, block, 0, stream>>>(
-        Q, kc, vc, pos, QG, ldp, O, ldo, T, Hq, Hkv, max_len, scale_log2, 1.f, xcd_split);
-  return hipGetLastError();
+  const size_t need = prefill_wide_ws_bytes(T, Hq, Hkv, max_len);
+  float* w = ws && need && ws_bytes >= need ? static_cast<float*>(ws) : nullptr;
+  return launch_prefill_wide(q, kc, vc, pos, qg, ldp, out, ldo, T, Hq, Hkv, max_len, scale * k_scale,
+                             kv8, v_scale, w, stream);
+}
+
+extern "C" size_t qe_attn_prefill_ws_size(int T, int Hq, int Hkv, int max_len) {
+  if (T < 1 || Hq < 1 || Hkv < 1 || Hq % Hkv != 0 || max_len < 1 || !prefill_wide_valid(T, Hq, Hkv) ||
+      balanced_grid(T, Hq, Hkv))
+    return 0;
+  return prefill_wide_ws_bytes(T, Hq, Hkv, max_len);
+}
+
+extern "C" hipError_t qe_attn_prefill_ws(const void* q, const void* kc, const void* vc,
+                                         const int* pos, const void* qg, long ldp, void* out,
+                                         long ldo, int T, int Hq, int Hkv, int max_len, float scale,
+                                         void* ws, size_t ws_bytes, hipStream_t stream) {
+  return launch_prefill(q, kc, vc, pos, qg, ldp, out, ldo, T, Hq, Hkv, max_len, scale, false, 1.f,
+                        1.f, ws, ws_bytes, stream);
 }
 
 extern "C" hipError_t qe_attn_prefill(const void* q, const void* kc, const void* vc,
                                       const int* pos, const void* qg, long ldp, void* out,
                                       long ldo, int T, int Hq, int Hkv, int max_len, float scale,
                                       hipStream_t stream) {
-  return launch_prefill(q, kc, vc, pos, qg, ldp, out, ldo, T, Hq, Hkv, max_len, scale, false, 1.f,
-                        1.f, stream);
+  return qe_attn_prefill_ws(q, kc, vc, pos, qg, ldp, out, ldo, T, Hq, Hkv, max_len, scale, nullptr, 0,
+                            stream);
+}
+
+extern "C" hipError_t qe_attn_prefill_fp8_ws(const void* q, const void* kc8, const void* vc8,
+                                             const int* pos, const void* qg, long ldp, void* out,
+                                             long ldo, int T, int Hq, int Hkv, int max_len,
+                                             float scale, float k_scale, float v_scale, void* ws,
+                                             size_t ws_bytes, hipStream_t stream) {
+  if (!kv_scale_ok(k_scale) || !kv_scale_ok(v_scale))
+    return hipErrorInvalidValue;
+  return launch_prefill(q, kc8, vc8, pos, qg, ldp, out, ldo, T, Hq, Hkv, max_len, scale, true,
+                        k_scale, v_scale, ws, ws_bytes, stream);
 }
 
 extern "C" hipError_t qe_attn_prefill_fp8(const void* q, const void* kc8, const void* vc8,
@@ -641,8 +466,6 @@ extern "C" hipError_t qe_attn_prefill_fp8(const void* q, const void* kc8, const 
                                           long ldo, int T, int Hq, int Hkv, int max_len,
                                           float scale, float k_scale, float v_scale,
                                           hipStream_t stream) {
-  if (!kv_scale_ok(k_scale) || !kv_scale_ok(v_scale))
-    return hipErrorInvalidValue;
-  return launch_prefill(q, kc8, vc8, pos, qg, ldp, out, ldo, T, Hq, Hkv, max_len, scale, true,
-                        k_scale, v_scale, stream);
+  return qe_attn_prefill_fp8_ws(q, kc8, vc8, pos, qg, ldp, out, ldo, T, Hq, Hkv, max_len, scale,
+                                k_scale, v_scale, nullptr, 0, stream);
 }

@@ -1,0 +1,19 @@
+// The prefill kernels of attn_prefill_wide.hip, launched from attn_prefill.hip.
+#pragma once
+#include <hip/hip_runtime.h>
+#include <stddef.h>
+
+namespace qe {
+
+// Whether the column and workgroup counts of a call fit 32 bits.
+bool prefill_wide_valid(int T, int Hq, int Hkv);
+// Workspace with which a call cuts units into slices; 0 where it never would.
+size_t prefill_wide_ws_bytes(int T, int Hq, int Hkv, int max_len);
+// ws: prefill_wide_ws_bytes() bytes, 16-byte aligned, or null (no slices). v_scale multiplies O / l
+// before its bf16 rounding (exactly 1 for the bf16 cache).
+hipError_t launch_prefill_wide(const void* q, const void* kc, const void* vc, const int* pos,
+                               const void* qg, long ldp, void* out, long ldo, int T, int Hq, int Hkv,
+                               int max_len, float scale, bool kv8, float v_scale, float* ws,
+                               hipStream_t stream);
+
+}  // namespace qe

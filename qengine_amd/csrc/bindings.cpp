@@ -1,7 +1,8 @@
 // torch bindings for qengine_amd._C: the reference's qengine._C attention ops with the same
 // Python signatures and the same validation contract (reference csrc/bindings.cpp:1-30,147-183).
-// Every op writes into caller-provided tensors (no allocation), enqueues on the current HIP stream
-// and never syncs, so it can be captured in a hipGraph. Row-batched arguments are 2-D views
+// Every op writes into caller-provided tensors, enqueues on the current HIP stream and never syncs,
+// so it can be captured in a hipGraph. None allocates, except the prefill ops outside a capture
+// (prefill_ws). Row-batched arguments are 2-D views
 // [n, width] with stride(1) == 1 and any row stride (a 1-D tensor counts as one row).
 //
 // Each op is a thin shell over the C ABI in include/qe_attn.h. Launch errors are raised as
@@ -217,13 +218,31 @@ PrefillArgs parse_prefill(const torch::Tensor& q, const torch::Tensor& kc, const
   return {T, Hq, Hkv, max_len, QG.ld, O.ld};
 }
 
+// Workspace of a prefill call from torch's allocator (its block is reused in stream order), or an
+// undefined tensor: where the call needs none, where memory is short, and under stream capture, since
+// a capture that is not torch's own would keep the address of a block that goes back to the pool.
+torch::Tensor prefill_ws(const PrefillArgs& a, const torch::Tensor& like, hipStream_t stream) {
+  const size_t bytes = qe_attn_prefill_ws_size(a.T, a.Hq, a.Hkv, a.max_len);
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  if (bytes == 0 || hipStreamIsCapturing(stream, &st) != hipSuccess ||
+      st != hipStreamCaptureStatusNone)
+    return {};
+  try {
+    return torch::empty({(int64_t)bytes}, like.options().dtype(torch::kByte));
+  } catch (const c10::OutOfMemoryError&) {
+    return {};
+  }
+}
+
 void attn_prefill(torch::Tensor q, torch::Tensor kc, torch::Tensor vc, torch::Tensor pos,
                   torch::Tensor qg, torch::Tensor out) {
   const auto a = parse_prefill(q, kc, vc, pos, qg, out, true);
   const c10::DeviceGuard guard(q.device());
-  raise_on(qe_attn_prefill(q.data_ptr(), kc.data_ptr(), vc.data_ptr(), pos.data_ptr<int>(),
-                           qg.data_ptr(), a.ldp, out.data_ptr(), a.ldo, a.T, a.Hq, a.Hkv,
-                           a.max_len, 1.0f / 16.0f, stream_of(q)),
+  const auto ws = prefill_ws(a, q, stream_of(q));
+  raise_on(qe_attn_prefill_ws(q.data_ptr(), kc.data_ptr(), vc.data_ptr(), pos.data_ptr<int>(),
+                              qg.data_ptr(), a.ldp, out.data_ptr(), a.ldo, a.T, a.Hq, a.Hkv,
+                              a.max_len, 1.0f / 16.0f, ws.defined() ? ws.data_ptr() : nullptr,
+                              ws.defined() ? ws.nbytes() : 0, stream_of(q)),
            "qe_attn_prefill");
 }
 
@@ -343,10 +362,12 @@ void attn_prefill_fp8(torch::Tensor q, torch::Tensor kc8, torch::Tensor vc8, tor
   kv_scales(k_scale, v_scale);
   const auto a = parse_prefill(q, kc8, vc8, pos, qg, out, true, true);
   const c10::DeviceGuard guard(q.device());
-  raise_on(qe_attn_prefill_fp8(q.data_ptr(), kc8.data_ptr(), vc8.data_ptr(), pos.data_ptr<int>(),
-                               qg.data_ptr(), a.ldp, out.data_ptr(), a.ldo, a.T, a.Hq, a.Hkv,
-                               a.max_len, 1.0f / 16.0f, (float)k_scale, (float)v_scale,
-                               stream_of(q)),
+  const auto ws = prefill_ws(a, q, stream_of(q));
+  raise_on(qe_attn_prefill_fp8_ws(q.data_ptr(), kc8.data_ptr(), vc8.data_ptr(), pos.data_ptr<int>(),
+                                  qg.data_ptr(), a.ldp, out.data_ptr(), a.ldo, a.T, a.Hq, a.Hkv,
+                                  a.max_len, 1.0f / 16.0f, (float)k_scale, (float)v_scale,
+                                  ws.defined() ? ws.data_ptr() : nullptr,
+                                  ws.defined() ? ws.nbytes() : 0, stream_of(q)),
            "qe_attn_prefill_fp8");
 }
 

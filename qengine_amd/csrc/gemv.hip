@@ -182,8 +182,7 @@ static hipError_t launch_gemv_xr(const __bf16* W, const __bf16* x, __bf16* out, 
   return hipGetLastError();
 }
 
-// Compute units of the current device (256 on MI355X; 256 when it cannot be queried).
-static int device_cus() {
+int compute_units() {
   static std::atomic<int> cache[64];
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
@@ -217,7 +216,7 @@ extern "C" int qe_gemv_tile_rows(int N, int K) {
   if (N < 1 || K < 1) return 0;
   // Only grids of one tile per workgroup (S = 4) and at most 4 workgroups per CU are re-cut:
   // with more rounds the part-empty last one is a small share of the call.
-  const long cus = device_cus();
+  const long cus = compute_units();
   if (qe_gemv_kparts(N, K) != 4 || (N + 15) / 16 > 4 * cus) return 16;
   // the tile height whose grid best fills its last round over the CUs; ties keep taller tiles
   int best = 16;

@@ -13,6 +13,9 @@ typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
 
+// Compute units of the current device (256 on MI355X; 256 when it cannot be queried). Host only.
+int compute_units();
+
 // ---------------------------------------------------------------------------- bf16 rounding
 // torch rounds every bf16 op result to nearest-even; these model one such rounding.
 __device__ __forceinline__ float bf16_to_f32(__bf16 x) { return static_cast<float>(x); }

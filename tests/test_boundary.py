@@ -588,3 +588,19 @@ def test_default_splits_policy():
     assert qa.default_splits(1000, 4, cus=256) == 32  # ceil(1000 / 32)
     assert qa.default_splits(64, 4, cus=256, kv8=True) == 2
     assert qa.default_splits(1, 64, cus=4) == 1
+
+
+def test_capi_prefill_workspace_size(capi):
+    """qe_attn_prefill_ws_size on 256 compute units: 0 for arguments that the call rejects, where the
+    units of 128 columns fill whole rounds, where the cache is too short for slices to pay and for the
+    balanced kernel's shapes; otherwise two slots per concurrent workgroup (O of 128 columns, max and
+    sum of its 256 lanes)."""
+    size = capi.load().qe_attn_prefill_ws_size
+    slots = 2 * 256 * (128 * D + 2 * 256) * 4
+    assert size(0, 24, 4, 4096) == 0 and size(16, 25, 4, 4096) == 0 and size(16, 24, 4, 0) == 0
+    assert size(301, 24, 4, 16384) == slots
+    assert size(9, 16, 2, 32768) == slots
+    assert size(2048, 32, 8, 8192) == 0   # 64 units of each KV head on 32 workgroups
+    assert size(40, 24, 4, 128) == 0
+    assert size(2048, 24, 4, 4096) == 0   # 256 balanced workgroups
+    assert size(2049, 24, 4, 4096) == slots
