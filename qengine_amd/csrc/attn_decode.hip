@@ -843,6 +843,31 @@ attn_partials_kernel(const __bf16* __restrict__ q, const __bf16* kc, const __bf1
       // and order as the NT >= 2 merge below, so the bits do not depend on NT.
       const int col = c;
       const bool mine = in_pass(col, grp, P);
+      // One tile: the other waves hold m = -inf, l = 0, O = 0, so wave 0's accumulators are the
+      // partial, bit for bit, and no barrier is needed. A short prefix is a chain of latencies, and
+      // the merge's two LDS passes were part of it: prep + decode of one row at 1k (24/4 heads)
+      // went from 10.4 to 9.6 us. (Conditions on the number of active waves inside the general
+      // sums, instead, put its LDS reads behind branches: 3% slower at 16k.)
+      if (P.end - P.beg <= TILE) {
+        if (w != 0 || !mine) return;
+        const int t = trow[0], head = g * grp + (col - t * grp);
+        const size_t slot = ((size_t)t * Hq + head) * NS + s;
+        if (g4 == 0) {
+          part_ml[slot * 2] = m[0];
+          part_ml[slot * 2 + 1] = l[0];
+        }
+        float* dst = part_o + slot * HD + 32 * g4;
+#pragma unroll
+        for (int hh = 0; hh < 2; ++hh)
+#pragma unroll
+          for (int ii = 0; ii < 4; ++ii)
+#pragma unroll
+            for (int i = 0; i < 8; i += 4)
+              *reinterpret_cast<f32x4_t*>(dst + 128 * hh + 8 * ii + i) =
+                  f32x4_t{acc[0][8 * hh + i][ii], acc[0][8 * hh + i + 1][ii],
+                          acc[0][8 * hh + i + 2][ii], acc[0][8 * hh + i + 3][ii]};
+        return;
+      }
       if (g4 == 0) {
         s_m[w][col] = m[0];
         s_l[w][col] = l[0];
@@ -851,7 +876,7 @@ attn_partials_kernel(const __bf16* __restrict__ q, const __bf16* kc, const __bf1
 #pragma unroll
         for (int a = 0; a < 16; ++a) s_acc(w, a) = acc[0][a];
       }
-      __syncthreads();
+      lds_barrier();
       if (!mine) return;
       float M = -INFINITY, wsc[WAVES];
 #pragma unroll
@@ -893,7 +918,7 @@ attn_partials_kernel(const __bf16* __restrict__ q, const __bf16* kc, const __bf1
         s_l[w][ct * 16 + c] = l[ct];
       }
     }
-    __syncthreads();  // also: every wave is done with its K tile, so `lds` can hold the merge
+    lds_barrier();  // also: every wave is done with its K tile, so `lds` can hold the merge
 
     float wsc[NT][WAVES];
 #pragma unroll
@@ -927,12 +952,12 @@ attn_partials_kernel(const __bf16* __restrict__ q, const __bf16* kc, const __bf1
     for (int ct = 0; ct < NT; ++ct) {
       const int col = ct * 16 + c;
       const bool mine = in_pass(col, grp, P);
-      if (ct > 0) __syncthreads();  // the previous column tile's reads are done
+      if (ct > 0) lds_barrier();  // the previous column tile's reads are done (its stores need not be)
       if (mine) {
 #pragma unroll
         for (int a = 0; a < 16; ++a) s_acc[w][a][lane] = acc[ct][a];
       }
-      __syncthreads();
+      lds_barrier();
       if (mine) {
         const int h = w >> 1, i0 = 4 * (w & 1);
         f32x4_t mo[4];
@@ -955,7 +980,7 @@ attn_partials_kernel(const __bf16* __restrict__ q, const __bf16* kc, const __bf1
   if (attendA) run_pass(PA, true);
   if constexpr (MULTI) {
     if (attendB) {
-      if (attendA) __syncthreads();  // the merge's LDS reads are done before the next pass
+      if (attendA) lds_barrier();  // the merge's LDS reads are done before the next pass
       run_pass(PB, !attendA);
     }
   }
@@ -993,17 +1018,8 @@ constexpr int STAGE8_U4 = TILE * HD / 16;  // 16-byte slots of one fp8 tile: 8 K
 // Two column tiles per wave already spill and keep the compiler's order.
 template <int CPW>
 constexpr int LEAD = CPW == 1 ? 4 : 0;
+constexpr int PLEAD = 4;  // qk_pairs and pv_pairs: operand reads in flight
 
-// 16 one-KB LDS-DMA loads of a bf16 K (or V) tile, rows 2i, 2i+1, shared by the subset's waves
-template <bool IS_V>
-__device__ __forceinline__ void issue_kv(__amdgpu_buffer_rsrc_t rs, int p0, u32x4_t* dst, int rank,
-                                         int wps, int lane) {
-  for (int i = rank; i < 16; i += wps) {
-    const int row = 2 * i + (lane >> 5);
-    const int q = IS_V ? (lane & 31) ^ tile::v_swz(row) : (lane & 31) ^ (row & 15);
-    buffer_load16_to_lds(rs, (uint32_t)(p0 + row) * (HD * 2) + q * 16, dst + 2 * i * ROW_CHUNKS);
-  }
-}
 // 8 one-KB LDS-DMA loads of an fp8 tile, rows 4i .. 4i+3, row-major (chunk q of row r at 16 r + q)
 __device__ __forceinline__ void issue_fp8(__amdgpu_buffer_rsrc_t rs, int p0, u32x4_t* dst, int rank,
                                           int wps, int lane) {
@@ -1012,38 +1028,133 @@ __device__ __forceinline__ void issue_fp8(__amdgpu_buffer_rsrc_t rs, int p0, u32
     buffer_load16_to_lds(rs, (uint32_t)(p0 + row) * HD + (lane & 15) * 16, dst + 64 * i);
   }
 }
-// LD: what the half loads (0 a bf16 V tile, 1 a bf16 K tile, 2 an fp8 tile)
-template <int LD>
-__device__ __forceinline__ void issue(__amdgpu_buffer_rsrc_t rs, int p, u32x4_t* dst, int rank,
-                                      int wps, int lane) {
-  if constexpr (LD == 2)
-    issue_fp8(rs, p, dst, rank, wps, lane);
-  else
-    issue_kv<LD == 0>(rs, p, dst, rank, wps, lane);
+// bf16 tiles of the bf16-cache kernels: rows in pairs of 1024 bytes plus a pad, row 2p + o at
+// PAIR p + 512 o. K's 16-byte chunks are XORed with o and V's 32-byte pieces with o, which spreads
+// the 16 rows of a K read and the 8 rows of a transposing V read over all banks with every address
+// one (K) or two (V) per-lane bases plus an immediate. (The XOR by row & 15 of tile::k_slot needs an
+// address per read, and with two column tiles a wave has no registers for them: it spilled 34 VGPRs,
+// the query among them, and could not afford the look-ahead rounds. Prep + decode of 8 rows at GQA 8,
+// 6k prefix: 27.3 -> 26.2 us.)
+constexpr int KPAIR = 2 * HD * 2 + 32, VPAIR = 2 * HD * 2 + 64;
+constexpr int KTILE_P = TILE / 2 * KPAIR, REGION_P = KTILE_P + TILE / 2 * VPAIR;  // bytes
+// 16 one-KB LDS-DMA loads (a row pair each) of a bf16 K (or V) tile, shared by the subset's waves.
+// rs starts at the tile's first row.
+template <bool IS_V>
+__device__ __forceinline__ void issue_pairs(__amdgpu_buffer_rsrc_t rs, char* dst, int rank, int wps,
+                                            int lane) {
+  const uint32_t o = lane >> 5, off = o * (HD * 2) + ((lane & 31) ^ (IS_V ? 2 * o : o)) * 16;
+  for (int i = rank; i < 16; i += wps)
+    buffer_load16_to_lds(rs, off + (uint32_t)i * (2 * HD * 2), dst + i * (IS_V ? VPAIR : KPAIR));
 }
-template <int CPW, int LD>
-__device__ __forceinline__ void qk_softmax_half(
-    const u32x4_t* __restrict__ kt, u32x4_t* __restrict__ dst, bool has, bool load, int p_load,
-    __amdgpu_buffer_rsrc_t rs, int p0, int Lmin, int rank, int wps, int lane, int c, int g4,
-    const bf16x8_t (&qb)[CPW][8], const int (&Lcol)[CPW], float scale_log2, float (&m)[CPW],
-    float (&l)[CPW], f32x4_t (&acc)[CPW][16], u32x4_t (&pb_hi)[CPW], u32x4_t (&pb_lo)[CPW]) {
-  if (load) issue<LD>(rs, p_load, dst, rank, wps, lane);
-  if (!has) return;
-  f32x4_t sacc[CPW][2];
-  tile::qk_tile<CPW, false, LEAD<CPW>>(kt, qb, c, g4, sacc);
+// S^T of a tile, tile::qk_tile's arithmetic: operand k = positions 16 (k >> 3) .., dims 32 (k & 7) ..;
+// LEAD reads run ahead of the MFMAs.
+template <int CPW>
+__device__ __forceinline__ void qk_pairs(const char* __restrict__ kt, const bf16x8_t (&qb)[CPW][8],
+                                         int lane, f32x4_t (&sacc)[CPW][2]) {
+  const int c = lane & 15, o = c & 1;
+  const char* k0 = kt + (c >> 1) * KPAIR + o * (HD * 2) + 16 * ((lane >> 4) ^ o);
+  auto read = [&](int k) __attribute__((always_inline)) {
+    return as_bf16x8(*reinterpret_cast<const u32x4_t*>(k0 + (k >> 3) * (8 * KPAIR) + 64 * (k & 7)));
+  };
+  bf16x8_t op[16];
+#pragma unroll
+  for (int k = 0; k < PLEAD; ++k) op[k] = read(k);
+#pragma unroll
+  for (int u = 0; u < CPW; ++u) sacc[u][0] = sacc[u][1] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int k = 0; k < 16; ++k) {
+#pragma unroll
+    for (int u = 0; u < CPW; ++u) sacc[u][k >> 3] = mfma16x16x32(op[k], qb[u][k & 7], sacc[u][k >> 3]);
+    if (k + PLEAD < 16) op[k + PLEAD] = read(k + PLEAD);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+}
+// O^T += V^T P^T of a tile, tile::pv_tile_tr's arithmetic (P as hi + lo terms).
+template <int CPW>
+__device__ __forceinline__ void pv_pairs(const char* __restrict__ vt, int lane,
+                                         const u32x4_t (&hi)[CPW], const u32x4_t (&lo)[CPW],
+                                         f32x4_t (&acc)[CPW][16]) {
+  typedef short v4i16 __attribute__((ext_vector_type(4)));
+  typedef __attribute__((address_space(3))) v4i16 lds_v4i16;
+  const int x = (lane >> 2) & 3, o = x & 1;  // rows 4 g4 + x and + 16, dims 16i + 4 (lane & 3) .. +3
+  const char* v0 = vt + (2 * (lane >> 4) + (x >> 1)) * VPAIR + o * (HD * 2) + 8 * (lane & 3);
+  const char* vb[2] = {v0 + 32 * o, v0 + 32 * (1 - o)};  // piece i of the row is at i ^ o
+  auto read = [&](int i) __attribute__((always_inline)) {
+    const char* a = vb[i & 1] + 32 * (i & 14);
+    const u32x2_t y = __builtin_bit_cast(u32x2_t, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4i16*)a));
+    const u32x2_t z = __builtin_bit_cast(
+        u32x2_t, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4i16*)(a + 8 * VPAIR)));
+    return as_bf16x8(u32x4_t{y[0], y[1], z[0], z[1]});
+  };
+  bf16x8_t op[16];
+#pragma unroll
+  for (int i = 0; i < PLEAD; ++i) op[i] = read(i);
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+#pragma unroll
+    for (int u = 0; u < CPW; ++u) {
+      acc[u][i] = mfma16x16x32(op[i], as_bf16x8(hi[u]), acc[u][i]);
+      acc[u][i] = mfma16x16x32(op[i], as_bf16x8(lo[u]), acc[u][i]);
+    }
+    if (i + PLEAD < 16) op[i + PLEAD] = read(i + PLEAD);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+}
+template <int CPW>
+__device__ __forceinline__ void softmax(const f32x4_t (&sacc)[CPW][2], int p0, int Lmin,
+                                        const int (&Lcol)[CPW], float scale_log2, int g4,
+                                        float (&m)[CPW], float (&l)[CPW], f32x4_t (&acc)[CPW][16],
+                                        u32x4_t (&pb_hi)[CPW], u32x4_t (&pb_lo)[CPW]) {
   if (p0 + TILE > Lmin)
     tile::softmax_tile<CPW, true, true>(sacc, p0, Lcol, scale_log2, g4, m, l, acc, pb_hi, pb_lo);
   else
     tile::softmax_tile<CPW, false, true>(sacc, p0, Lcol, scale_log2, g4, m, l, acc, pb_hi, pb_lo);
 }
-template <int CPW, int LD>
+// The two halves of a look-ahead round on the bf16 cache: what one half loads is never what it reads.
+template <int CPW>
+__device__ __forceinline__ void half_s(const char* __restrict__ kt, char* __restrict__ vt, bool has,
+                                       bool load, __amdgpu_buffer_rsrc_t vrs, int p0, int Lmin,
+                                       int rank, int wps, int lane, const bf16x8_t (&qb)[CPW][8],
+                                       const int (&Lcol)[CPW], float scale_log2, float (&m)[CPW],
+                                       float (&l)[CPW], f32x4_t (&acc)[CPW][16],
+                                       u32x4_t (&pb_hi)[CPW], u32x4_t (&pb_lo)[CPW]) {
+  if (load) issue_pairs<true>(vrs, vt, rank, wps, lane);
+  if (!has) return;
+  f32x4_t sacc[CPW][2];
+  qk_pairs<CPW>(kt, qb, lane, sacc);
+  softmax<CPW>(sacc, p0, Lmin, Lcol, scale_log2, lane >> 4, m, l, acc, pb_hi, pb_lo);
+}
+template <int CPW>
+__device__ __forceinline__ void half_o(const char* __restrict__ vt, char* __restrict__ kt, bool has,
+                                       bool load, __amdgpu_buffer_rsrc_t krs, int rank, int wps,
+                                       int lane, const u32x4_t (&pb_hi)[CPW],
+                                       const u32x4_t (&pb_lo)[CPW], f32x4_t (&acc)[CPW][16]) {
+  if (load) issue_pairs<false>(krs, kt, rank, wps, lane);
+  if (has) pv_pairs<CPW>(vt, lane, pb_hi, pb_lo, acc);
+}
+// The fp8 cache's halves: each loads an fp8 tile into the staging buffer.
+template <int CPW>
+__device__ __forceinline__ void qk_softmax_half(
+    const u32x4_t* __restrict__ kt, u32x4_t* __restrict__ dst, bool has, bool load, int p_load,
+    __amdgpu_buffer_rsrc_t rs, int p0, int Lmin, int rank, int wps, int lane, int c, int g4,
+    const bf16x8_t (&qb)[CPW][8], const int (&Lcol)[CPW], float scale_log2, float (&m)[CPW],
+    float (&l)[CPW], f32x4_t (&acc)[CPW][16], u32x4_t (&pb_hi)[CPW], u32x4_t (&pb_lo)[CPW]) {
+  if (load) issue_fp8(rs, p_load, dst, rank, wps, lane);
+  if (!has) return;
+  f32x4_t sacc[CPW][2];
+  tile::qk_tile<CPW, false, LEAD<CPW>>(kt, qb, c, g4, sacc);
+  softmax<CPW>(sacc, p0, Lmin, Lcol, scale_log2, g4, m, l, acc, pb_hi, pb_lo);
+}
+template <int CPW>
 __device__ __forceinline__ void pv_half_la(const u32x4_t* __restrict__ vt,
                                            u32x4_t* __restrict__ dst, bool has, bool load,
                                            int p_load, __amdgpu_buffer_rsrc_t rs, int rank,
                                            int wps, int lane, int g4,
                                            const u32x4_t (&pb_hi)[CPW], const u32x4_t (&pb_lo)[CPW],
                                            f32x4_t (&acc)[CPW][16]) {
-  if (load) issue<LD>(rs, p_load, dst, rank, wps, lane);
+  if (load) issue_fp8(rs, p_load, dst, rank, wps, lane);
   if (has) tile::pv_tile_tr<CPW, true, false, LEAD<CPW>>(vt, lane, g4, pb_hi, pb_lo, acc);
 }
 // All NTH threads of the workgroup convert the fp8 tiles of the first nact subsets once, from
@@ -1098,7 +1209,9 @@ attn_partials_cols_kernel(const __bf16* __restrict__ q, const __bf16* __restrict
   const int s = blockIdx.x, g = blockIdx.y;
   const int grp = Hq / Hkv;
   const int lane = threadIdx.x & (WAVE - 1), w = threadIdx.x / WAVE;
-  const int sub = w % SUB, rank = w / SUB;
+  // A subset's waves are consecutive, so that slices with fewer tiles than subsets still spread over
+  // the SIMDs (wave w runs on SIMD w mod 4).
+  const int sub = w / WPS, rank = w % WPS;
   const int c = lane & 15, g4 = lane >> 4;
   const int ncols = grp * n;
 
@@ -1130,8 +1243,8 @@ attn_partials_cols_kernel(const __bf16* __restrict__ q, const __bf16* __restrict
   // buffer (4 x 40 KB: all 160 KB of LDS), and s_m / s_l live in the ring past the merge's two
   // accumulator buffers (the ring is idle once the rounds end).
   constexpr bool LA8 = KV8 && CPW == 1;
-  constexpr int REGION = LA8 ? cols::REGION_U4 + cols::STAGE8_U4 : cols::REGION_U4;
-  __shared__ __attribute__((aligned(16))) u32x4_t lds[SUB * REGION];  // 128 KB or 160 KB
+  constexpr int REGION = !KV8 ? cols::REGION_P / 16 : LA8 ? cols::REGION_U4 + cols::STAGE8_U4 : cols::REGION_U4;
+  __shared__ __attribute__((aligned(16))) u32x4_t lds[SUB * REGION];  // 134 KB (bf16), 128 or 160 KB
   __shared__ float s_m_[LA8 ? 1 : SUB][16 * NT], s_l_[LA8 ? 1 : SUB][16 * NT];
   static_assert(!LA8 || 2 * SUB * 16 * WAVE * 16 + 2 * SUB * 16 * NT * 4 <= SUB * REGION * 16,
                 "s_m and s_l fit the ring past the two merge buffers");
@@ -1144,10 +1257,11 @@ attn_partials_cols_kernel(const __bf16* __restrict__ q, const __bf16* __restrict
   u32x4_t* kt = lds + sub * REGION;
   u32x4_t* vt = kt + cols::TILE_U4;
   u32x4_t* st = vt + cols::TILE_U4;  // LA8: the fp8 staging buffer
+  char *kp = reinterpret_cast<char*>(kt), *vp = kp + cols::KTILE_P;  // bf16 cache
 
   // One pass, inlined once per call of the lambda (a loop over passes would keep the merge's
   // loop-invariant addresses live through the tile rounds and spill).
-  auto run_pass = [&](const Pass P) __attribute__((always_inline)) {
+  auto run_pass = [&](const Pass P, bool more) __attribute__((always_inline)) {
     int Lcol[CPW];
 #pragma unroll
     for (int u = 0; u < CPW; ++u)
@@ -1171,15 +1285,16 @@ attn_partials_cols_kernel(const __bf16* __restrict__ q, const __bf16* __restrict
 
     const int ntiles = (P.end - P.beg + TILE - 1) / TILE;
     const int rounds = (ntiles + SUB - 1) / SUB;
-    if constexpr (!KV8 && CPW == 1) {
-      // Two barriers per round as before (one when the pass has one round); each one also
-      // publishes the tile loaded during the half-round before it. (CPW = 2 keeps the loop below:
-      // there the look-ahead's longer-lived addresses add spills, 30 -> 70, and it ran 17-42%
-      // slower at GQA 8.)
+    if constexpr (!KV8) {
+      // Two barriers per round (one when the pass has one round); each one also publishes the tile
+      // loaded during the half-round before it.
+      const auto rsrc = [&](const __bf16* base, int p) __attribute__((always_inline)) {
+        return tile_rsrc(reinterpret_cast<const char*>(base) + head_off, p, P.end, HD * 2);
+      };
       const int p00 = P.beg + sub * TILE;
       if (p00 < P.end) {
-        cols::issue_kv<false>(krs, p00, kt, rank, WPS, lane);
-        cols::issue_kv<true>(vrs, p00, vt, rank, WPS, lane);
+        cols::issue_pairs<false>(rsrc(kc, p00), kp, rank, WPS, lane);
+        cols::issue_pairs<true>(rsrc(vc, p00), vp, rank, WPS, lane);
       }
       vmcnt_wait<0>();
       __syncthreads();  // K and V of round 0 have landed
@@ -1189,15 +1304,14 @@ attn_partials_cols_kernel(const __bf16* __restrict__ q, const __bf16* __restrict
         const int p1 = p0 + SUB * TILE;
         const bool has1 = r + 1 < rounds && p1 < P.end;
         u32x4_t pb_hi[CPW], pb_lo[CPW];
-        cols::qk_softmax_half<CPW, 0>(kt, vt, has, has && r > 0, p0, vrs, p0, P.Lmin, rank, WPS,
-                                      lane, c, g4, qb, Lcol, scale_log2, m, l, acc, pb_hi, pb_lo);
+        cols::half_s<CPW>(kp, vp, has, has && r > 0, rsrc(vc, p0), p0, P.Lmin, rank, WPS, lane, qb,
+                          Lcol, scale_log2, m, l, acc, pb_hi, pb_lo);
         // (The wait stays outside the branch: behind a join the compiler's wait-count pass
         // assumes V may still be in flight and waits for the K load below before PV.)
         vmcnt_wait<0>();
         if (r > 0 || r + 1 < rounds)  // uniform
           __syncthreads();  // V of round r has landed; K of round r is no longer read
-        cols::pv_half_la<CPW, 1>(vt, kt, has, has1, p1, krs, rank, WPS, lane, g4, pb_hi, pb_lo,
-                                 acc);
+        cols::half_o<CPW>(vp, kp, has, has1, rsrc(kc, p1), rank, WPS, lane, pb_hi, pb_lo, acc);
         vmcnt_wait<0>();
         __syncthreads();  // K of round r+1 has landed; V of round r is no longer read
       }
@@ -1226,7 +1340,7 @@ attn_partials_cols_kernel(const __bf16* __restrict__ q, const __bf16* __restrict
         const bool more = r + 1 < rounds;                // uniform
         const bool has1 = more && p1 < P.end;
         u32x4_t pb_hi[CPW], pb_lo[CPW];
-        cols::qk_softmax_half<CPW, 2>(kt, st, has, has1, p1, krs, p0, P.Lmin, rank, WPS, lane, c,
+        cols::qk_softmax_half<CPW>(kt, st, has, has1, p1, krs, p0, P.Lmin, rank, WPS, lane, c,
                                       g4, qb, Lcol, scale_log2, m, l, acc, pb_hi, pb_lo);
         // (The waits stay outside the branches: behind a join the compiler's wait-count pass
         // would assume a load in flight and wait for the next one before the operand reads.)
@@ -1236,7 +1350,7 @@ attn_partials_cols_kernel(const __bf16* __restrict__ q, const __bf16* __restrict
           cols::convert_fp8<false, NTH>(lds, REGION, 2 * cols::TILE_U4, 0, nact(r + 1));
           __syncthreads();  // bf16 K of round r+1 whole; the staging buffer is free
         }
-        cols::pv_half_la<CPW, 2>(vt, st, has, has1, p1, vrs, rank, WPS, lane, g4, pb_hi, pb_lo,
+        cols::pv_half_la<CPW>(vt, st, has, has1, p1, vrs, rank, WPS, lane, g4, pb_hi, pb_lo,
                                  acc);
         vmcnt_wait<0>();
         __syncthreads();  // fp8 V of round r+1 has landed; bf16 V of round r is no longer read
@@ -1249,25 +1363,13 @@ attn_partials_cols_kernel(const __bf16* __restrict__ q, const __bf16* __restrict
     for (int r = 0; r < rounds; ++r) {
       const int p0 = P.beg + (r * SUB + sub) * TILE;  // this subset's tile in round r
       const bool has = p0 < P.end;                     // uniform per subset
-      if (has && KV8) {
+      if (has) {
         // fp8: 8 loads of K then 8 of V, one KB (rows 4j .. 4j+3) each, shared by the subset's
         // waves: 16-byte chunk q of row r of K at vt[16 r + q], of V at vt[512 + 16 r + q].
         for (int i = rank; i < 16; i += WPS) {
           const int row = 4 * (i & 7) + (lane >> 4);
           buffer_load16_to_lds(i < 8 ? krs : vrs, (uint32_t)(p0 + row) * HD + (lane & 15) * 16,
                                vt + 64 * i);
-        }
-      } else if (has) {
-        // The subset's WPS waves share its 32 LDS-DMA loads: 16 of K (rows 2i, 2i+1, swizzled as
-        // k_slot) and 16 of V (swizzled as tile::v_swz), one KB of contiguous cache each.
-        for (int i = rank; i < 32; i += WPS) {
-          const int j = i & 15, row = 2 * j + (lane >> 5);
-          if (i < 16)
-            buffer_load16_to_lds(krs, (uint32_t)(p0 + row) * (HD * 2) + ((lane & 31) ^ (row & 15)) * 16,
-                                 kt + 2 * j * ROW_CHUNKS);
-          else
-            buffer_load16_to_lds(vrs, (uint32_t)(p0 + row) * (HD * 2) + ((lane & 31) ^ tile::v_swz(row)) * 16,
-                                 kt + cols::TILE_U4 + 2 * j * ROW_CHUNKS);
         }
       }
       vmcnt_wait<0>();
@@ -1325,7 +1427,9 @@ attn_partials_cols_kernel(const __bf16* __restrict__ q, const __bf16* __restrict
       __syncthreads();  // this round's tiles are read before the next round overwrites them
     }
 
-    // ---- merge the 4 subsets in order 0..3 (as attn_partials_kernel merges its waves)
+    // ---- merge the 4 subsets in order 0..3 (as attn_partials_kernel merges its waves). Subsets
+    // without a tile hold m = -inf, l = 0, O = 0: with at most two tiles the terms of subsets 2 and 3
+    // (weight 0) stay out, which changes no bit. The barriers order LDS alone, not the stores.
 #pragma unroll
     for (int u = 0; u < CPW; ++u) {
       l[u] = group4_sum(l[u]);
@@ -1334,7 +1438,7 @@ attn_partials_cols_kernel(const __bf16* __restrict__ q, const __bf16* __restrict
         s_l[sub][(rank * CPW + u) * 16 + c] = l[u];
       }
     }
-    __syncthreads();
+    lds_barrier();
     float wsc[CPW][SUB];
 #pragma unroll
     for (int u = 0; u < CPW; ++u) {
@@ -1365,45 +1469,53 @@ attn_partials_cols_kernel(const __bf16* __restrict__ q, const __bf16* __restrict
     static_assert(GROUP * SUB * 16 * WAVE * 16 <= SUB * cols::REGION_U4 * 16,
                   "two items' merge buffers fit the ring");
     f32x4_t (*s_acc)[SUB][16][WAVE] = reinterpret_cast<f32x4_t (*)[SUB][16][WAVE]>(lds);
+    auto merge = [&](auto na) __attribute__((always_inline)) {
+      constexpr int NA = decltype(na)::value;
 #pragma unroll
-    for (int i0 = 0; i0 < NI; i0 += GROUP) {
+      for (int i0 = 0; i0 < NI; i0 += GROUP) {
 #pragma unroll
-      for (int gi = 0; gi < GROUP; ++gi) {
-        if (i0 + gi >= NI) break;
-        const int u = (i0 + gi) / WPS, rr = (i0 + gi) % WPS;
-        if (rank == rr && in_pass((rr * CPW + u) * 16 + c, grp, P)) {
+        for (int gi = 0; gi < GROUP; ++gi) {
+          if (i0 + gi >= NI) break;
+          const int u = (i0 + gi) / WPS, rr = (i0 + gi) % WPS;
+          if (rank == rr && sub < NA && in_pass((rr * CPW + u) * 16 + c, grp, P)) {
 #pragma unroll
-          for (int a = 0; a < 16; ++a) s_acc[gi][sub][a][lane] = acc[u][a];
-        }
-      }
-      __syncthreads();
-#pragma unroll
-      for (int gi = 0; gi < GROUP; ++gi) {
-        if (i0 + gi >= NI) break;
-        const int u = (i0 + gi) / WPS, rr = (i0 + gi) % WPS;
-        const int col = (rr * CPW + u) * 16 + c;
-        if (rank == rr && in_pass(col, grp, P)) {
-          f32x4_t mo[4];
-#pragma unroll
-          for (int k = 0; k < 4; ++k) {
-            f32x4_t sum = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int v = 0; v < SUB; ++v) sum += s_acc[gi][v][4 * sub + k][lane] * wsc[u][v];
-            mo[k] = sum;
+            for (int a = 0; a < 16; ++a) s_acc[gi][sub][a][lane] = acc[u][a];
           }
-          const int t = col / grp, head = g * grp + (col - t * grp);
-          float* dst = part_o + (((size_t)t * Hq + head) * NS + s) * HD;
-          // acc[i][k] = O^T[16i + 4g4 + k] (tile::pv_tile_tr)
-#pragma unroll
-          for (int k = 0; k < 4; ++k)
-            reinterpret_cast<f32x4_t*>(dst + 16 * (4 * sub + k) + 4 * g4)[0] = mo[k];
         }
+        lds_barrier();
+#pragma unroll
+        for (int gi = 0; gi < GROUP; ++gi) {
+          if (i0 + gi >= NI) break;
+          const int u = (i0 + gi) / WPS, rr = (i0 + gi) % WPS;
+          const int col = (rr * CPW + u) * 16 + c;
+          if (rank == rr && in_pass(col, grp, P)) {
+            f32x4_t mo[4];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+              f32x4_t sum = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+              for (int v = 0; v < NA; ++v) sum += s_acc[gi][v][4 * sub + k][lane] * wsc[u][v];
+              mo[k] = sum;
+            }
+            const int t = col / grp, head = g * grp + (col - t * grp);
+            float* dst = part_o + (((size_t)t * Hq + head) * NS + s) * HD;
+            // acc[i][k] = O^T[16i + 4g4 + k] (tile::pv_tile_tr)
+#pragma unroll
+            for (int k = 0; k < 4; ++k)
+              reinterpret_cast<f32x4_t*>(dst + 16 * (4 * sub + k) + 4 * g4)[0] = mo[k];
+          }
+        }
+        if (more || i0 + GROUP < NI) lds_barrier();  // (also ends the pass: the next one loads over `lds`)
       }
-      __syncthreads();  // (also ends the pass: the next pass's loads may overwrite `lds`)
-    }
+    };
+    if (CPW == 1 && ntiles <= 2)
+      merge(std::integral_constant<int, 2>{});
+    else
+      merge(std::integral_constant<int, SUB>{});
   };
-  if (attendA) run_pass(PA);
-  if (npass > 1 && PB.beg < PB.end) run_pass(PB);
+  const bool attendB = npass > 1 && PB.beg < PB.end;
+  if (attendA) run_pass(PA, attendB);
+  if (attendB) run_pass(PB, false);
 }
 
 static bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
