@@ -17,8 +17,8 @@ constexpr int GDN_THREADS = 1024;                   // one-workgroup kernel: 16 
 constexpr int GDN_SPLIT = 4;                        // workgroups per head in the split kernel
 constexpr int GDN_SPLIT_COLS = GDN_D / GDN_SPLIT;
 constexpr int GDN_SPLIT_THREADS = 512;
+constexpr int GDN_FINISH_THREADS = 512;
 constexpr int GDN_SPLIT_MIN_ROWS = 5;               // fewer rows: the one-workgroup kernel
-constexpr int GDN_STAGE_MAX_ROWS = 2;               // up to this many: the state staged in LDS
 
 struct __align__(16) F4 {
   float x, y, z, w;
@@ -75,10 +75,22 @@ __device__ __forceinline__ void read_out(const float (&s)[8][NC], const float (&
   for (int c = 0; c < NC; ++c) o[c] = round_bf16(colquad_sum(o[c]));
 }
 
+// x at position P + r of channel ch: a row of this call (r >= n re-reads row n - 1) or the ring.
+__device__ __forceinline__ __bf16 conv_input(const __bf16* __restrict__ qkv, long ldp,
+                                             const __bf16* ring, int C, int P, int n, int r,
+                                             int ch) {
+  return *(r >= 0 ? qkv + (size_t)min(r, n - 1) * ldp + ch
+                  : ring + (size_t)((P + r) & (GDN_RING - 1)) * C + ch);
+}
+// What the conv reads there: zero before the sequence.
+__device__ __forceinline__ float conv_value(__bf16 x, int P, int r) {
+  return r >= 0 || P + r >= 0 ? bf16_to_f32(x) : 0.f;
+}
 // Causal conv (4 taps, the HF buffer order [x_{t-3}, x_{t-2}, x_{t-1}, x_t]) and SiLU of row t of
-// one channel; xs holds x at positions P-3 .. P+n-1. Rounds to bf16 after the conv and after SiLU.
-__device__ __forceinline__ float conv_silu(const float (&cw)[4], const float (&xs)[3 + GDN_MAXN],
-                                           int t) {
+// one channel; xs[t .. t+3] holds x at positions P+t-3 .. P+t. Rounds to bf16 after the conv and
+// after SiLU.
+template <int N>
+__device__ __forceinline__ float conv_silu(const float (&cw)[4], const float (&xs)[N], int t) {
   float acc = cw[0] * xs[t];
   acc = fmaf(cw[1], xs[t + 1], acc);
   acc = fmaf(cw[2], xs[t + 2], acc);
@@ -98,55 +110,12 @@ __device__ __forceinline__ void lds_read8(const float* p, float (&d)[8]) {
   const F4 a = *reinterpret_cast<const F4*>(p), b = *reinterpret_cast<const F4*>(p + 4);
   d[0] = a.x; d[1] = a.y; d[2] = a.z; d[3] = a.w; d[4] = b.x; d[5] = b.y; d[6] = b.z; d[7] = b.w;
 }
-__device__ __forceinline__ void lds_read4(const float* p, float (&d)[4]) {
-  const F4 a = *reinterpret_cast<const F4*>(p);
-  d[0] = a.x; d[1] = a.y; d[2] = a.z; d[3] = a.w;
-}
-// NC consecutive floats (NC = 1, 2 or 4), LDS or global memory: one vector access for 2 or 4.
-template <int NC>
-__device__ __forceinline__ void vec_read_n(const float* p, float (&d)[NC]) {
-  if constexpr (NC == 4) {
-    lds_read4(p, d);
-  } else if constexpr (NC == 2) {
-    const float2 a = *reinterpret_cast<const float2*>(p);
-    d[0] = a.x; d[1] = a.y;
-  } else {
-#pragma unroll
-    for (int c = 0; c < NC; ++c) d[c] = p[c];
-  }
-}
-template <int NC>
-__device__ __forceinline__ void vec_write_n(float* p, const float (&d)[NC]) {
-  if constexpr (NC == 4) {
-    *reinterpret_cast<F4*>(p) = F4{d[0], d[1], d[2], d[3]};
-  } else if constexpr (NC == 2) {
-    *reinterpret_cast<float2*>(p) = make_float2(d[0], d[1]);
-  } else {
-#pragma unroll
-    for (int c = 0; c < NC; ++c) p[c] = d[c];
-  }
-}
-// This lane's block of a head's state (rows 8 rg .. +7, columns col0 .. col0 + NC - 1 of the
-// row-major [128][128] fp32 state): 8 loads of 4 NC bytes, and the write-back.
-template <int NC>
-__device__ __forceinline__ void load_state_rows(const float* Sj, int rg, int col0,
-                                                float (&s)[8][NC]) {
-#pragma unroll
-  for (int rr = 0; rr < 8; ++rr) vec_read_n(Sj + (size_t)(rg * 8 + rr) * GDN_D + col0, s[rr]);
-}
-template <int NC>
-__device__ __forceinline__ void store_state_rows(float* Sj, int rg, int col0,
-                                                 const float (&s)[8][NC]) {
-#pragma unroll
-  for (int rr = 0; rr < 8; ++rr) vec_write_n(Sj + (size_t)(rg * 8 + rr) * GDN_D + col0, s[rr]);
-}
-
 // Gated RMSNorm of one output row of a head (wave-wide; lane holds columns 2 lane, 2 lane + 1):
 // out = bf16(bf16(w * bf16(o * r)) * silu(z)), r = 1 / sqrt(sum(o^2) / 128 + eps). The sum of
 // squares is four serial 32-column partials added in order, the same in every kernel, so every
 // path gives the same bits.
 __device__ __forceinline__ void gated_norm_row(const float* __restrict__ o_row, int lane, float nw0,
-                                               float nw1, float z0, float z1, float eps,
+                                               float nw1, float silu_z0, float silu_z1, float eps,
                                                __bf16* __restrict__ op) {
   const float2 o = *reinterpret_cast<const float2*>(&o_row[2 * lane]);
   float part_ss = 0.f;
@@ -163,8 +132,8 @@ __device__ __forceinline__ void gated_norm_row(const float* __restrict__ o_row, 
   const float inv = 1.0f / sqrtf(ss / 128.0f + eps);
   const float y0 = round_bf16(nw0 * round_bf16(o.x * inv));  // bf16 weight * bf16 norm
   const float y1 = round_bf16(nw1 * round_bf16(o.y * inv));
-  op[2 * lane] = f32_to_bf16(y0 * silu_f(z0));
-  op[2 * lane + 1] = f32_to_bf16(y1 * silu_f(z1));
+  op[2 * lane] = f32_to_bf16(y0 * silu_z0);
+  op[2 * lane + 1] = f32_to_bf16(y1 * silu_z1);
 }
 
 // Split path for 5-8 rows (gdn_split.hip): gdn_split_kernel then gdn_finish_kernel.
