@@ -1206,6 +1206,7 @@ attn_partials_cols_kernel(const __bf16* __restrict__ q, const __bf16* __restrict
   constexpr int SUB = cols::SUBSETS;
   constexpr int WPS = NT / CPW;  // waves per subset
   const int pos0 = pos_ptr[0] + row0;  // first: the slicing waits for it
+  asm volatile("" ::: "memory");       // (and it is not sunk below the query's loads)
   const int s = blockIdx.x, g = blockIdx.y;
   const int grp = Hq / Hkv;
   const int lane = threadIdx.x & (WAVE - 1), w = threadIdx.x / WAVE;
@@ -1262,11 +1263,17 @@ attn_partials_cols_kernel(const __bf16* __restrict__ q, const __bf16* __restrict
   // One pass, inlined once per call of the lambda (a loop over passes would keep the merge's
   // loop-invariant addresses live through the tile rounds and spill).
   auto run_pass = [&](const Pass P, bool more) __attribute__((always_inline)) {
+    // The columns' attended lengths, computed once the first tile's loads are out: what is reloaded
+    // for them (the registers are few) waits for every load before it, the query's first of all.
     int Lcol[CPW];
+    auto lcol = [&]() __attribute__((always_inline)) {
+      int cc = c;
+      asm volatile("" : "+v"(cc));
 #pragma unroll
-    for (int u = 0; u < CPW; ++u)
-      Lcol[u] = in_pass((rank * CPW + u) * 16 + c, grp, P)
-                    ? min(pos0 + ((rank * CPW + u) * 16 + c) / grp + 1, max_len) : 0;
+      for (int u = 0; u < CPW; ++u)
+        Lcol[u] = in_pass((rank * CPW + u) * 16 + cc, grp, P)
+                      ? min(pos0 + ((rank * CPW + u) * 16 + cc) / grp + 1, max_len) : 0;
+    };
     const uint32_t bytes = (uint32_t)P.end * (uint32_t)(HD * ELEM);
     const __amdgpu_buffer_rsrc_t krs =
         make_rsrc_uniform(reinterpret_cast<const char*>(kc) + head_off, bytes);
@@ -1296,6 +1303,7 @@ attn_partials_cols_kernel(const __bf16* __restrict__ q, const __bf16* __restrict
         cols::issue_pairs<false>(rsrc(kc, p00), kp, rank, WPS, lane);
         cols::issue_pairs<true>(rsrc(vc, p00), vp, rank, WPS, lane);
       }
+      lcol();
       vmcnt_wait<0>();
       __syncthreads();  // K and V of round 0 have landed
       for (int r = 0; r < rounds; ++r) {
@@ -1327,6 +1335,7 @@ attn_partials_cols_kernel(const __bf16* __restrict__ q, const __bf16* __restrict
         cols::issue_fp8(krs, p00, st, rank, WPS, lane);
         cols::issue_fp8(vrs, p00, kt + cols::STAGE8_U4, rank, WPS, lane);
       }
+      lcol();
       vmcnt_wait<0>();
       __syncthreads();  // the fp8 tiles of round 0 have landed
       cols::convert_fp8<true, NTH>(lds, REGION, cols::STAGE8_U4, cols::TILE_U4, nact(0));
@@ -1361,6 +1370,7 @@ attn_partials_cols_kernel(const __bf16* __restrict__ q, const __bf16* __restrict
       }
     } else
     for (int r = 0; r < rounds; ++r) {
+      if (r == 0) lcol();
       const int p0 = P.beg + (r * SUB + sub) * TILE;  // this subset's tile in round r
       const bool has = p0 < P.end;                     // uniform per subset
       if (has) {
