@@ -26,7 +26,12 @@ namespace qe {
 // maximum, and the gate's sigmoid computed while the partials are in flight. Layer-call, 1 row at
 // 16k: 17.9 us with the earlier form, 16.8 with this one (32- and 64-dim chunks of the same
 // design: 17.0 and 17.6; 16-dim was also the fastest or within 0.3% at 2-8 rows).
+// VEC: gate and output rows are 8-byte aligned, so a lane's 4 dims are one access instead of four
+// (prep + decode of one row, 24 / 4 heads: 1k 9.66 -> 9.61 us per layer, twice; longer calls unchanged).
+// The loads of a second batch of 64 slices issued ahead of the first batch's sums measured slower:
+// 8 rows on 6k positions at 16 / 2 heads, 94 slices, 25.2 -> 25.4 us per layer.
 constexpr int COMBINE_DIMS = 16;
+typedef __bf16 bf16x4_t __attribute__((ext_vector_type(4)));
 
 // Sum / max over the 16 lane groups of 4 lanes: lane ^ 32, ^ 16 (the gfx950 lane swaps), ^ 8
 // and ^ 4 (DPP within each 16-lane row) pair group g with g ^ 8, g ^ 4, g ^ 2, g ^ 1. Every lane
@@ -42,6 +47,7 @@ __device__ __forceinline__ float group16_max(float v) {
   return xor32_pair(xor16_pair(v, false), false);
 }
 
+template <bool VEC>
 __global__ void __launch_bounds__(WAVE)
 attn_combine_kernel(const float* __restrict__ part_o, const float* __restrict__ part_ml,
                     const int* __restrict__ pos_ptr, const __bf16* __restrict__ qg, long ldp,
@@ -55,9 +61,13 @@ attn_combine_kernel(const float* __restrict__ part_o, const float* __restrict__ 
   const int dim = z * COMBINE_DIMS + 4 * cd;
   const __bf16* gp = qg + (size_t)t * ldp + (size_t)h * 2 * HD + HD + dim;
 
-  float gate[4];  // qg rows carry no alignment guarantee beyond 2 bytes
+  bf16x4_t gate;
+  if constexpr (VEC) {
+    gate = *reinterpret_cast<const bf16x4_t*>(gp);
+  } else {
 #pragma unroll
-  for (int i = 0; i < 4; ++i) gate[i] = bf16_to_f32(gp[i]);
+    for (int i = 0; i < 4; ++i) gate[i] = gp[i];
+  }
   __builtin_amdgcn_sched_barrier(0);  // the gate's load is issued first
   // The first batch of slices is loaded before pos arrives (every slot below NS exists in the
   // caller's buffers); slots past row t's slice count S are discarded by selection, so stale
@@ -77,7 +87,7 @@ attn_combine_kernel(const float* __restrict__ part_o, const float* __restrict__ 
   float sgate[4];  // bf16(sigmoid(gate)), computed while the partials are in flight
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    sgate[i] = round_bf16(sigmoid_f32(gate[i]));
+    sgate[i] = round_bf16(sigmoid_f32(bf16_to_f32(gate[i])));
     asm volatile("" : "+v"(sgate[i]));  // here, not sunk to the stores
   }
   const int L_t = min(pos_ptr[0] + t + 1, max_len);
@@ -116,11 +126,18 @@ attn_combine_kernel(const float* __restrict__ part_o, const float* __restrict__ 
   for (int i = 0; i < 4; ++i) O[i] = group16_sum(O[i]);
   if (g == 0) {
     __bf16* op = out + (size_t)t * ldo + (size_t)h * HD + dim;
+    bf16x4_t r;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       // attention output is a bf16 tensor (v_scale: the fp8 cache's V scale, else exactly 1)
       const float o = round_bf16((O[i] / L) * v_scale);
-      op[i] = f32_to_bf16(o * sgate[i]);
+      r[i] = f32_to_bf16(o * sgate[i]);
+    }
+    if constexpr (VEC) {
+      *reinterpret_cast<bf16x4_t*>(op) = r;
+    } else {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) op[i] = r[i];
     }
   }
 }
@@ -128,7 +145,10 @@ attn_combine_kernel(const float* __restrict__ part_o, const float* __restrict__ 
 hipError_t launch_combine(const float* part_o, const float* part_ml, const int* pos,
                           const void* qg, long ldp, void* out, long ldo, int n, int Hq,
                           int max_len, int NS, hipStream_t stream, float v_scale) {
-  attn_combine_kernel<<<dim3(Hq, n, HD / COMBINE_DIMS), dim3(WAVE), 0, stream>>>(
+  const bool vec = ((reinterpret_cast<uintptr_t>(qg) | reinterpret_cast<uintptr_t>(out)) & 7) == 0 &&
+                   ldp % 4 == 0 && ldo % 4 == 0;
+  auto kern = vec ? attn_combine_kernel<true> : attn_combine_kernel<false>;
+  kern<<<dim3(Hq, n, HD / COMBINE_DIMS), dim3(WAVE), 0, stream>>>(
       part_o, part_ml, pos, static_cast<const __bf16*>(qg), ldp, static_cast<__bf16*>(out), ldo,
       Hq, max_len, NS, ns_div(NS), v_scale);
   return hipGetLastError();
