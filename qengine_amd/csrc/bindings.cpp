@@ -218,6 +218,20 @@ PrefillArgs parse_prefill(const torch::Tensor& q, const torch::Tensor& kc, const
   return {T, Hq, Hkv, max_len, QG.ld, O.ld};
 }
 
+// This thread's capture interaction mode, relaxed for a scope. With the default mode a device
+// allocation is refused while any thread captures a stream in the global mode, and refusing it ends
+// that thread's capture too.
+struct RelaxedCaptureMode {
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  RelaxedCaptureMode() { hip_ok(hipThreadExchangeStreamCaptureMode(&mode)); }
+  ~RelaxedCaptureMode() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+  RelaxedCaptureMode(const RelaxedCaptureMode&) = delete;
+  RelaxedCaptureMode& operator=(const RelaxedCaptureMode&) = delete;
+
+ private:
+  static void hip_ok(hipError_t e) { TORCH_CHECK(e == hipSuccess, hipGetErrorString(e)); }
+};
+
 // Workspace of a prefill call from torch's allocator (its block is reused in stream order), or an
 // undefined tensor: where the call needs none, where memory is short, and under stream capture, since
 // a capture that is not torch's own would keep the address of a block that goes back to the pool.
@@ -228,6 +242,7 @@ torch::Tensor prefill_ws(const PrefillArgs& a, const torch::Tensor& like, hipStr
       st != hipStreamCaptureStatusNone)
     return {};
   try {
+    const RelaxedCaptureMode relaxed;  // another thread may be capturing
     return torch::empty({(int64_t)bytes}, like.options().dtype(torch::kByte));
   } catch (const c10::OutOfMemoryError&) {
     return {};
