@@ -1032,19 +1032,28 @@ __device__ __forceinline__ void issue_fp8(__amdgpu_buffer_rsrc_t rs, int p0, u32
 // PAIR p + 512 o. K's 16-byte chunks are XORed with o and V's 32-byte pieces with o, which spreads
 // the 16 rows of a K read and the 8 rows of a transposing V read over all banks with every address
 // one (K) or two (V) per-lane bases plus an immediate. (The XOR by row & 15 of tile::k_slot needs an
-// address per read, and with two column tiles a wave has no registers for them: it spilled 34 VGPRs,
-// the query among them, and could not afford the look-ahead rounds. Prep + decode of 8 rows at GQA 8,
-// 6k prefix: 27.3 -> 26.2 us.)
+// address per read, and with two column tiles a wave has no registers for them.)
 constexpr int KPAIR = 2 * HD * 2 + 32, VPAIR = 2 * HD * 2 + 64;
 constexpr int KTILE_P = TILE / 2 * KPAIR, REGION_P = KTILE_P + TILE / 2 * VPAIR;  // bytes
 // 16 one-KB LDS-DMA loads (a row pair each) of a bf16 K (or V) tile, shared by the subset's waves.
-// rs starts at the tile's first row.
-template <bool IS_V>
-__device__ __forceinline__ void issue_pairs(__amdgpu_buffer_rsrc_t rs, char* dst, int rank, int wps,
-                                            int lane) {
-  const uint32_t o = lane >> 5, off = o * (HD * 2) + ((lane & 31) ^ (IS_V ? 2 * o : o)) * 16;
-  for (int i = rank; i < 16; i += wps)
-    buffer_load16_to_lds(rs, off + (uint32_t)i * (2 * HD * 2), dst + i * (IS_V ? VPAIR : KPAIR));
+// rs starts at the tile's first row. dst, the tile's LDS byte address, and rank, the wave in the subset,
+// are in scalar registers, so that M0 is scalar arithmetic. The lane offsets are made anew for every
+// tile (opaque to the compiler): hoisted out of the rounds they are a register per load, which the
+// kernel of two column tiles per wave has to spill, and the reload of a spilled offset waits for the
+// load before it. us per call, loop without look-ahead / offsets hoisted (41 VGPRs spilled) / now (none): 8
+// rows at 16 / 2 heads on 6k 25.0 / 22.8 / 22.5, 16k 31.4 / 33.6 / 26.8, 64k 52.2 / 64.9 / 42.4; three column
+// tiles, 8 rows at 24 / 4 on 64k 60.2 / 60.8 / 57.2. (The pair's place is not in the instruction's scalar
+// offset, which the range check leaves out.)
+template <bool IS_V, int WPS>
+__device__ __forceinline__ void issue_pairs(__amdgpu_buffer_rsrc_t rs, uint32_t dst, int rank, int lane) {
+  const uint32_t o = lane >> 5;
+  uint32_t off = o * (HD * 2) + ((lane & 31) ^ (IS_V ? 2 * o : o)) * 16 + rank * (2 * HD * 2);
+  asm volatile("" : "+v"(off));
+  dst += rank * (IS_V ? VPAIR : KPAIR);
+#pragma unroll
+  for (int k = 0; k < (16 + WPS - 1) / WPS; ++k)
+    if (16 % WPS == 0 || k * WPS + rank < 16)
+      buffer_load16_to_lds_at(rs, off + k * (WPS * 2 * HD * 2), dst + k * (WPS * (IS_V ? VPAIR : KPAIR)));
 }
 // S^T of a tile, tile::qk_tile's arithmetic: operand k = positions 16 (k >> 3) .., dims 32 (k & 7) ..;
 // LEAD reads run ahead of the MFMAs.
@@ -1113,25 +1122,24 @@ __device__ __forceinline__ void softmax(const f32x4_t (&sacc)[CPW][2], int p0, i
     tile::softmax_tile<CPW, false, true>(sacc, p0, Lcol, scale_log2, g4, m, l, acc, pb_hi, pb_lo);
 }
 // The two halves of a look-ahead round on the bf16 cache: what one half loads is never what it reads.
-template <int CPW>
-__device__ __forceinline__ void half_s(const char* __restrict__ kt, char* __restrict__ vt, bool has,
+template <int CPW, int WPS>
+__device__ __forceinline__ void half_s(const char* __restrict__ kt, uint32_t vt, bool has,
                                        bool load, __amdgpu_buffer_rsrc_t vrs, int p0, int Lmin,
-                                       int rank, int wps, int lane, const bf16x8_t (&qb)[CPW][8],
+                                       int rank, int lane, const bf16x8_t (&qb)[CPW][8],
                                        const int (&Lcol)[CPW], float scale_log2, float (&m)[CPW],
                                        float (&l)[CPW], f32x4_t (&acc)[CPW][16],
                                        u32x4_t (&pb_hi)[CPW], u32x4_t (&pb_lo)[CPW]) {
-  if (load) issue_pairs<true>(vrs, vt, rank, wps, lane);
+  if (load) issue_pairs<true, WPS>(vrs, vt, rank, lane);
   if (!has) return;
   f32x4_t sacc[CPW][2];
   qk_pairs<CPW>(kt, qb, lane, sacc);
   softmax<CPW>(sacc, p0, Lmin, Lcol, scale_log2, lane >> 4, m, l, acc, pb_hi, pb_lo);
 }
-template <int CPW>
-__device__ __forceinline__ void half_o(const char* __restrict__ vt, char* __restrict__ kt, bool has,
-                                       bool load, __amdgpu_buffer_rsrc_t krs, int rank, int wps,
-                                       int lane, const u32x4_t (&pb_hi)[CPW],
+template <int CPW, int WPS>
+__device__ __forceinline__ void half_o(const char* __restrict__ vt, uint32_t kt, bool has,
+                                       bool load, __amdgpu_buffer_rsrc_t krs, int rank, int lane, const u32x4_t (&pb_hi)[CPW],
                                        const u32x4_t (&pb_lo)[CPW], f32x4_t (&acc)[CPW][16]) {
-  if (load) issue_pairs<false>(krs, kt, rank, wps, lane);
+  if (load) issue_pairs<false, WPS>(krs, kt, rank, lane);
   if (has) pv_pairs<CPW>(vt, lane, pb_hi, pb_lo, acc);
 }
 // The fp8 cache's halves: each loads an fp8 tile into the staging buffer.
@@ -1209,7 +1217,8 @@ attn_partials_cols_kernel(const __bf16* __restrict__ q, const __bf16* __restrict
   asm volatile("" ::: "memory");       // (and it is not sunk below the query's loads)
   const int s = blockIdx.x, g = blockIdx.y;
   const int grp = Hq / Hkv;
-  const int lane = threadIdx.x & (WAVE - 1), w = threadIdx.x / WAVE;
+  const int lane = threadIdx.x & (WAVE - 1);
+  const int w = KV8 ? (int)(threadIdx.x / WAVE) : __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
   // A subset's waves are consecutive, so that slices with fewer tiles than subsets still spread over
   // the SIMDs (wave w runs on SIMD w mod 4).
   const int sub = w / WPS, rank = w % WPS;
@@ -1259,6 +1268,7 @@ attn_partials_cols_kernel(const __bf16* __restrict__ q, const __bf16* __restrict
   u32x4_t* vt = kt + cols::TILE_U4;
   u32x4_t* st = vt + cols::TILE_U4;  // LA8: the fp8 staging buffer
   char *kp = reinterpret_cast<char*>(kt), *vp = kp + cols::KTILE_P;  // bf16 cache
+  const uint32_t kl = KV8 ? 0 : lds_byte_uniform(kt);
 
   // One pass, inlined once per call of the lambda (a loop over passes would keep the merge's
   // loop-invariant addresses live through the tile rounds and spill).
@@ -1300,8 +1310,8 @@ attn_partials_cols_kernel(const __bf16* __restrict__ q, const __bf16* __restrict
       };
       const int p00 = P.beg + sub * TILE;
       if (p00 < P.end) {
-        cols::issue_pairs<false>(rsrc(kc, p00), kp, rank, WPS, lane);
-        cols::issue_pairs<true>(rsrc(vc, p00), vp, rank, WPS, lane);
+        cols::issue_pairs<false, WPS>(rsrc(kc, p00), kl, rank, lane);
+        cols::issue_pairs<true, WPS>(rsrc(vc, p00), kl + cols::KTILE_P, rank, lane);
       }
       lcol();
       vmcnt_wait<0>();
@@ -1312,14 +1322,14 @@ attn_partials_cols_kernel(const __bf16* __restrict__ q, const __bf16* __restrict
         const int p1 = p0 + SUB * TILE;
         const bool has1 = r + 1 < rounds && p1 < P.end;
         u32x4_t pb_hi[CPW], pb_lo[CPW];
-        cols::half_s<CPW>(kp, vp, has, has && r > 0, rsrc(vc, p0), p0, P.Lmin, rank, WPS, lane, qb,
-                          Lcol, scale_log2, m, l, acc, pb_hi, pb_lo);
+        cols::half_s<CPW, WPS>(kp, kl + cols::KTILE_P, has, has && r > 0, rsrc(vc, p0), p0, P.Lmin, rank,
+                               lane, qb, Lcol, scale_log2, m, l, acc, pb_hi, pb_lo);
         // (The wait stays outside the branch: behind a join the compiler's wait-count pass
         // assumes V may still be in flight and waits for the K load below before PV.)
         vmcnt_wait<0>();
         if (r > 0 || r + 1 < rounds)  // uniform
           __syncthreads();  // V of round r has landed; K of round r is no longer read
-        cols::half_o<CPW>(vp, kp, has, has1, rsrc(kc, p1), rank, WPS, lane, pb_hi, pb_lo, acc);
+        cols::half_o<CPW, WPS>(vp, kl, has, has1, rsrc(kc, p1), rank, lane, pb_hi, pb_lo, acc);
         vmcnt_wait<0>();
         __syncthreads();  // K of round r+1 has landed; V of round r is no longer read
       }
