@@ -163,9 +163,13 @@ struct Convert {
   }
 };
 
-// sigmoid(x) by the hardware exponential and reciprocal (each within 1 ulp of fp32)
+// bf16(sigmoid_f32(x)) for a bf16 x, the same bits for all 65,536 of them (checked on MI355X), by the
+// hardware exponential and reciprocal. The reciprocal flushes subnormal results, so it is taken of
+// (1 + e) 2^-24 and scaled back: gates below -87.3 are subnormal, not 0.
 __device__ __forceinline__ float gate(float x) {
-  return round_bf16(__builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(-1.4426950408889634f * x)));
+  constexpr float s = 0x1p-24f;
+  const float e = __builtin_amdgcn_exp2f(-1.4426950408889634f * x);
+  return round_bf16(__builtin_amdgcn_rcpf(__builtin_fmaf(e, s, s)) * s);
 }
 
 struct State {

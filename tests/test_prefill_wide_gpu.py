@@ -114,3 +114,25 @@ def test_negative_scale(capi):
     assert capi.prefill(-q.to(DEV), kd, vd, p, *args, b, hq * D, T, hq, hkv, pos + T, 1.0 / 16) == 0
     torch.cuda.synchronize()
     assert torch.isfinite(a.float()).all() and torch.equal(a, b)
+
+
+@pytest.mark.parametrize("pos", [0, 3000])  # one pass over the cache, and slices
+def test_every_gate(native, pos):
+    """All 65,536 bf16 gates: with K = 0 and V = 1 the attention is exactly 1, and the output is the
+    gate's sigmoid. The decode op evaluates it by the library's exponential and a division; the prefill
+    has the same bits (-87.5 .. -88.5 give subnormal values)."""
+    hq, hkv, T = 16, 2, 16
+    gates = torch.arange(65536, dtype=torch.int32).to(torch.int16).view(BF).view(T, hq, 1, D)
+    qg = torch.cat([torch.zeros_like(gates), gates], 2).reshape(T, -1).to(DEV)
+    kc = torch.zeros(hkv, pos + T, D, dtype=BF, device=DEV)
+    q, vc = torch.zeros(T, hq * D, dtype=BF, device=DEV), torch.ones_like(kc)
+    out, ref = torch.empty_like(q), torch.empty_like(q)
+    p = torch.tensor([pos], dtype=torch.int32, device=DEV)
+    native.attn_prefill(q, kc, vc, p, qg, out)
+    po, pml = torch.empty(8, hq, 16, D, device=DEV), torch.empty(8, hq, 16, 2, device=DEV)
+    for t in (0, 8):
+        native.attn_decode(q[t:t + 8], kc, vc, p + t, qg[t:t + 8], po, pml, ref[t:t + 8])
+    nan = ref.isnan()
+    assert torch.equal(out.isnan(), nan)
+    assert torch.equal(out.view(torch.int16)[~nan], ref.view(torch.int16)[~nan])
+    assert ((ref > 0) & (ref.float() < 1.17e-38)).any()
