@@ -172,6 +172,18 @@ __device__ __forceinline__ float gate(float x) {
   return round_bf16(__builtin_amdgcn_rcpf(__builtin_fmaf(e, s, s)) * s);
 }
 
+// acc / L to within 2^-22 of a half ulp of the correctly rounded quotient, as two products: 1 / L is
+// hi + lo with lo > 0, so that infinities and NaN come out as a division gives them.
+struct Quotient {
+  float hi, lo;
+  __device__ __forceinline__ explicit Quotient(float L) {
+    const float r = 1.f / L;
+    hi = r > 0.f ? __uint_as_float(__float_as_uint(r) - 1) : r;
+    lo = fmaxf(__builtin_fmaf(-L, hi, 1.f) * r, 1.17549435e-38f);
+  }
+  __device__ __forceinline__ float operator()(float acc) const { return __builtin_fmaf(acc, hi, acc * lo); }
+};
+
 struct State {
   float m, l;
   f32x16_t acc[8];  // acc[i][r] = O^T[32i + 8(r>>2) + 4h + (r&3)][column c]
@@ -553,7 +565,12 @@ attn_prefill_wide_kernel(const __bf16* __restrict__ q, const void* __restrict__ 
     __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
                                      (lds_void*)(uintptr_t)(gt + 1024 * t), 16, 0, 0);
   }
-  const float inv = s.v_scale / L;
+  const Quotient by(L);
+  const auto o2 = [&](int i, int r) __attribute__((always_inline)) {  // two values of O as bf16
+    float a = by(st.acc[i][r]), b = by(st.acc[i][r + 1]);
+    if constexpr (KV8) a *= s.v_scale, b *= s.v_scale;
+    return pack_bf16x2(a, b);
+  };
   typedef __attribute__((address_space(3))) u32x2_t lds_u32x2;
   const uint32_t wr = ob + c * ROW_B + 8 * h;
 #pragma unroll
@@ -561,8 +578,7 @@ attn_prefill_wide_kernel(const __bf16* __restrict__ q, const void* __restrict__ 
 #pragma unroll
     for (int b = 0; b < 4; ++b)
       *(lds_u32x2*)(uintptr_t)(wr + 64 * i + 16 * b) =
-          u32x2_t{pack_bf16x2(st.acc[i][4 * b] * inv, st.acc[i][4 * b + 1] * inv),
-                  pack_bf16x2(st.acc[i][4 * b + 2] * inv, st.acc[i][4 * b + 3] * inv)};
+          u32x2_t{o2(i, 4 * b), o2(i, 4 * b + 2)};
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   vmcnt_wait<0>();
 #pragma unroll 2
@@ -630,11 +646,11 @@ attn_prefill_wide_combine(const int* __restrict__ pos_ptr, const __bf16* __restr
     }
     m = mn;
   }
-  const float inv = s.v_scale / L;
+  const Quotient by(L);
   uint32_t x[4];
 #pragma unroll
   for (int k = 0; k < 4; ++k)
-    x[k] = pack_bf16x2(o[k >> 1][2 * (k & 1)] * inv, o[k >> 1][2 * (k & 1) + 1] * inv);
+    x[k] = pack_bf16x2(by(o[k >> 1][2 * (k & 1)]) * s.v_scale, by(o[k >> 1][2 * (k & 1) + 1]) * s.v_scale);
   // both halves of the column's 8-dim block: lane half h gets block h
   const auto e0 = __builtin_amdgcn_permlane32_swap(x[0], x[2], false, false);
   const auto e1 = __builtin_amdgcn_permlane32_swap(x[1], x[3], false, false);

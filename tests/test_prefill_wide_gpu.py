@@ -136,3 +136,39 @@ def test_every_gate(native, pos):
     assert torch.equal(out.isnan(), nan)
     assert torch.equal(out.view(torch.int16)[~nan], ref.view(torch.int16)[~nan])
     assert ((ref > 0) & (ref.float() < 1.17e-38)).any()
+
+
+@pytest.mark.parametrize("sliced", [False, True])
+def test_least_v_scale(native, capi, sliced):
+    """O / L is rounded before V's scale multiplies it: the scale's least values (1.2e-38) give the bits
+    of a scale 2^100 times as large, times 2^-100, although scale / L would be subnormal."""
+    hq, hkv, T, pos = 16, 2, 16, 12000
+    g = gen(9)
+    q = torch.randn(T, hq * D, generator=g).to(BF).to(DEV)
+    kc = torch.randn(hkv, pos + T, D, generator=g).to(torch.float8_e4m3fn).to(DEV)
+    vc = (1 + 400 * torch.rand(hkv, pos + T, D, generator=g)).to(torch.float8_e4m3fn).to(DEV)
+    qg = torch.full((T, hq * 2 * D), 60.0, dtype=BF, device=DEV)  # gates of 1
+    p = torch.tensor([pos], dtype=torch.int32, device=DEV)
+    scale = torch.tensor(1.2e-38, dtype=torch.float32).item()
+    outs = []
+    for vs in (scale, scale * 2.0 ** 100):
+        out = torch.empty_like(q)
+        if sliced:
+            native.attn_prefill_fp8(q, kc, vc, p, qg, out, 1.0, vs)
+        else:
+            assert capi.prefill_fp8(q, kc, vc, p, qg, qg.stride(0), out, hq * D, T, hq, hkv, pos + T,
+                                    1.0, vs) == 0
+        outs.append(out.double())
+    assert outs[0].min() > 1.18e-38  # normal values
+    assert torch.equal(outs[0], outs[1] * 2.0 ** -100)
+
+
+def test_infinite_v(native):
+    """An infinity in V comes out as an infinity where the rows attend it with weight (one bf16 term of
+    P: beyond 512 positions), as from a division; dims without one are not touched."""
+    q, kc, vc, qg = inputs(6, 1, 40, 1040, 4)
+    vc[0, 3, 5], vc[0, 4, 9] = float("inf"), float("-inf")
+    out = run(native.attn_prefill, q, kc, vc, 1000, torch.zeros_like(qg)).float().view(40, 6, D)
+    assert (out[:, :, 5] == float("inf")).all() and (out[:, :, 9] == float("-inf")).all()
+    out[:, :, 5] = out[:, :, 9] = 0
+    assert torch.isfinite(out).all()
