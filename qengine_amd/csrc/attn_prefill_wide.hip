@@ -36,7 +36,10 @@ using tile::BN;
 constexpr int WAVES = 4;                        // one per SIMD
 constexpr int WCOLS = 32;                       // query columns per wave
 constexpr int UCOLS = WAVES * WCOLS;            // query columns of a unit (a workgroup)
-constexpr int SPLIT_BELOW = 512;
+// P takes two bf16 terms (hi + lo) where a row of a wave is in a block of 16 rows (a multiple of 16 on)
+// whose first row attends fewer positions than this: the rows that the balanced kernel, a block per
+// wave, gives two terms, and for the rest of the wave no fewer.
+constexpr int SPLIT_BELOW = 512, SPLIT_ROWS = 16;
 // LDS tiles: rows in pairs of 1024 bytes. K: row 2p + o at 1056 p + 512 o, its 16-byte chunks
 // XORed with o, so that 16 rows at one chunk cover all banks; every operand read is one per-lane
 // base plus an immediate. V: row 2p + o at 1152 p + 512 o, its 64-byte pieces XORed with o, so that
@@ -507,7 +510,7 @@ attn_prefill_wide_kernel(const __bf16* __restrict__ q, const void* __restrict__ 
       run_tiles<KV8, decltype(mk)::value, decltype(sp)::value>(j0, j1, rg, cv, base, Lcol, lane, qb,
                                                                s.scale_log2, kop, sc, st);
     };
-    if (Lmin < SPLIT_BELOW) {
+    if (min(pos0 + r0 / SPLIT_ROWS * SPLIT_ROWS + 1, s.max_len) < SPLIT_BELOW) {
       run(K_{}, V_{}, J0, jm);
       run(V_{}, V_{}, jm, je);
     } else {

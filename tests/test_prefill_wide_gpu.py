@@ -172,3 +172,24 @@ def test_infinite_v(native):
     assert (out[:, :, 5] == float("inf")).all() and (out[:, :, 9] == float("-inf")).all()
     out[:, :, 5] = out[:, :, 9] = 0
     assert torch.isfinite(out).all()
+
+
+@pytest.mark.parametrize("hq,hkv", [(24, 4), (8, 2), (4, 4)])
+def test_rows_of_two_term_blocks(native, hq, hkv):
+    """P keeps two bf16 terms for every row of a 16-row block that begins below 512 attended positions,
+    whatever rows a wave holds: rows 400 .. 415 of a chunk at position 103 (504 .. 519 positions) are
+    within fp32 sums of the exact attention, so that nearly every output is its bf16 rounding. (One term
+    is 2e-3 off, more than half of bf16's spacing for about two values in five.)"""
+    T, pos = 416, 103
+    q, kc, vc, qg = inputs(hq, hkv, T, pos + T, 5)
+    out = run(native.attn_prefill, q, kc, vc, pos, torch.full_like(qg, 60.0))  # gates of 1
+    rows, grp = range(400, 416), hq // hkv
+    K, V, Q = kc.double(), vc.double(), q.view(T, hq, D).double()
+    same = []
+    for r in rows:
+        L = pos + r + 1
+        for h in range(hq):
+            p = torch.softmax(K[h // grp, :L] @ Q[r, h] / 16, 0)
+            same.append(out.view(T, hq, D)[r, h] == (p @ V[h // grp, :L]).to(BF))
+    share = torch.stack(same).float().mean(1).view(len(rows), hq).mean(1)
+    assert share.min() > 0.99, share
