@@ -122,6 +122,10 @@ hipError_t qe_attn_prefill_ws(const void* q, const void* kc, const void* vc, con
                               int max_len, float scale, void* ws, size_t ws_bytes,
                               hipStream_t stream);
 
+/* 1 where such a prefill call (kv8: on an fp8 cache; ws: with a workspace of the size above) runs the
+ * kernel that pairs long and short row blocks, 0 where it runs the one of 32 columns per wave. */
+int qe_attn_prefill_balanced(int T, int Hq, int Hkv, int max_len, int kv8, int ws);
+
 /* Number of cache positions per split-KV slice for a row attending L positions with NS partial
  * slots: ceil(L/NS) rounded up to a multiple of 32 (at least 32); row t's partial s covers
  * positions [s*size, (s+1)*size) of [0, L). The reference cuts ceil(L/NS) (csrc/attn.cu:78-80);

@@ -32,6 +32,7 @@ SIGNATURES = {
     "qe_attn_prefill_fp8_ws": (_I, [_P, _P, _P, _P, _P, _L, _P, _L, _I, _I, _I, _I, _F, _F, _F, _P,
                                     _Z, _P]),
     "qe_attn_prefill_ws_size": (_Z, [_I, _I, _I, _I]),
+    "qe_attn_prefill_balanced": (_I, [_I, _I, _I, _I, _I, _I]),
     "qe_attn_prefill_fp8": (_I, [_P, _P, _P, _P, _P, _L, _P, _L, _I, _I, _I, _I, _F, _F, _F, _P]),
     "qe_attn_prep_decode": (_I, [_P, _P, _P, _L, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _L, _I, _I,
                                  _I, _I, _I, _I, _F, _F, _P]),

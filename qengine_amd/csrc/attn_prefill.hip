@@ -6,8 +6,8 @@
 //
 // Two kernels; launch_prefill chooses:
 //  * attn_prefill_wide_kernel (attn_prefill_wide.hip): any shape.
-//  * attn_prefill_bal_kernel (here): GQA 6 where its 16-row blocks of all heads fill one round of the
-//    CUs (T about 2,048 at 24 / 4 heads). 12 waves (three per SIMD) of one KV head own three quads of
+//  * attn_prefill_bal_kernel (here): GQA 6 where its 16-row blocks of all heads fill the CUs and the
+//    wide kernel's units do not (T about 2,048 at 24 / 4 heads; balanced_grid). 12 waves (three per SIMD) of one KV head own three quads of
 //    (16-row block, q head) units, four units of one length per quad, one unit of each quad per
 //    SIMD; the quads of a workgroup mix lengths so that every workgroup carries about the same work.
 //
@@ -376,17 +376,31 @@ attn_prefill_bal_kernel(const __bf16* __restrict__ q, const void* __restrict__ k
 
 using namespace qe;
 
-// The balanced kernel's grid, if it takes the call: GQA 6 and between 96% and all of the CUs in one
-// round of workgroups. Measured at 24 / 4 heads, us per call (one process, in turn), balanced
-// against wide: 2,048 rows on 0 / 2,048 / 12,000 positions 73 / 158 / 573 against 70 / 166 / 594 (bf16
-// cache), 78 / 166 / 595 against 76 / 183 / 636 (fp8); 1,970 rows on 2,048 154 against 161. With more
-// rows (a second round) or fewer (idle CUs) the wide kernel wins: 3,000 rows on 1,000 245 against
-// 191, 1,500 on 1,000 92 against 80.
-static int balanced_grid(int T, int Hq, int Hkv) {
+// The balanced kernel's grid if it takes the call, else 0: GQA 6 where its estimated time is less than
+// the wide kernel's (prefill_wide_steps, in whose unit it is), at the last chunk that fits the cache:
+// the position is known to the device alone, and a wide call's lead is largest on a short prefix, so
+// a call that runs wide is the faster one wherever it stands. A round of 256 workgroups takes 1.48 (bf16
+// cache) or 1.37 (fp8) steps for a tile of the prefix plus 0.6 of the chunk, and 35 or 30 outside the
+// tile loop; a part-empty last round nearly as much. Against both kernels timed at 24 / 4, 6 / 1, 12 / 2 and
+// 48 / 8 heads, 256 to 16,384 rows on 0 to 16,000 positions, both caches, with and without slices, the
+// choice at the call's own position costs 0.1% on average and 6% at most (1,960 rows of an empty fp8
+// cache). us per call, balanced / wide in slices / wide unsliced, 24 / 4 heads:
+//   bf16, 2,048 rows on 4,000: 241 / 247 / 264, 1,500 on 4,000 198 / 180 / 233, 4,096 on 16,000 1,584 / - / 1,564
+//   fp8, 2,048 rows on 4,000: 252 / 274 / 305, 1,500 on 4,000 221 / 203 / 270, 4,096 on 16,000 1,629 / - / 1,717
+static int balanced_grid(int T, int Hq, int Hkv, int max_len, bool kv8, bool ws) {
   if (Hq != prefill::BAL_GRP * Hkv) return 0;
   const long wgs = ((T + 15) / 16 + 1) / 2 * (long)Hkv;
+  if (wgs > 0x7fffffffL) return 0;
   const int cus = compute_units();
-  return wgs <= cus && wgs * 25 >= cus * 24L ? (int)wgs : 0;
+  const float pos = (float)(max_len > T ? max_len - T : 0);
+  const float round = (kv8 ? 1.37f : 1.48f) * (pos + 0.6f * (float)T) / tile::BN + (kv8 ? 30.f : 35.f);
+  const float part = (float)(wgs % cus) / (float)cus;
+  const float steps = round * ((float)(wgs / cus) + (part > 0.f ? 0.9f + 0.1f * part : 0.f));
+  return steps < prefill_wide_steps(T, Hq, Hkv, max_len, kv8, ws) ? (int)wgs : 0;
+}
+
+static bool prefill_shape_ok(int T, int Hq, int Hkv, int max_len) {
+  return T >= 1 && Hq >= 1 && Hkv >= 1 && Hq % Hkv == 0 && max_len >= 1 && prefill_wide_valid(T, Hq, Hkv);
 }
 
 static hipError_t launch_prefill(const void* q, const void* kc, const void* vc, const int* pos,
@@ -394,16 +408,16 @@ static hipError_t launch_prefill(const void* q, const void* kc, const void* vc, 
                                  int Hkv, int max_len, float scale, bool kv8, float k_scale,
                                  float v_scale, void* ws, size_t ws_bytes, hipStream_t stream) {
   auto a16 = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
-  if (T < 1 || Hq < 1 || Hkv < 1 || Hq % Hkv != 0 || max_len < 1 || !pos ||
-      !prefill_wide_valid(T, Hq, Hkv))
-    return hipErrorInvalidValue;
+  if (!prefill_shape_ok(T, Hq, Hkv, max_len) || !pos) return hipErrorInvalidValue;
   if (!a16(q) || !a16(kc) || !a16(vc) || !a16(qg) || !a16(out) || !a16(ws) || ldp % 8 != 0 ||
       ldo % 8 != 0)
     return hipErrorInvalidValue;
   // byte offsets of the tiles loaded past the last attended row fit the 32-bit buffer range
   if ((unsigned long long)(max_len + 5 * tile::BN) * HD * 2 >= (1ull << 32))
     return hipErrorInvalidValue;
-  if (const int grid = balanced_grid(T, Hq, Hkv)) {
+  const size_t need = prefill_wide_ws_bytes(T, Hq, Hkv, max_len);
+  float* w = ws && need && ws_bytes >= need ? static_cast<float*>(ws) : nullptr;
+  if (const int grid = balanced_grid(T, Hq, Hkv, max_len, kv8, w != nullptr)) {
     // KV-head-per-XCD placement when the heads divide the XCDs evenly and every XCD of a head gets
     // the same number of workgroups
     const int per_head = prefill::XCDS % Hkv == 0 ? prefill::XCDS / Hkv : 0;
@@ -421,17 +435,19 @@ static hipError_t launch_prefill(const void* q, const void* kc, const void* vc, 
           Q, kc, vc, pos, QG, ldp, O, ldo, T, Hq, Hkv, max_len, scale_log2, 1.f, xs);
     return hipGetLastError();
   }
-  const size_t need = prefill_wide_ws_bytes(T, Hq, Hkv, max_len);
-  float* w = ws && need && ws_bytes >= need ? static_cast<float*>(ws) : nullptr;
   return launch_prefill_wide(q, kc, vc, pos, qg, ldp, out, ldo, T, Hq, Hkv, max_len, scale * k_scale,
                              kv8, v_scale, w, stream);
 }
 
 extern "C" size_t qe_attn_prefill_ws_size(int T, int Hq, int Hkv, int max_len) {
-  if (T < 1 || Hq < 1 || Hkv < 1 || Hq % Hkv != 0 || max_len < 1 || !prefill_wide_valid(T, Hq, Hkv) ||
-      balanced_grid(T, Hq, Hkv))
-    return 0;
+  if (!prefill_shape_ok(T, Hq, Hkv, max_len) || balanced_grid(T, Hq, Hkv, max_len, false, true)) return 0;
   return prefill_wide_ws_bytes(T, Hq, Hkv, max_len);
+}
+
+extern "C" int qe_attn_prefill_balanced(int T, int Hq, int Hkv, int max_len, int kv8, int ws) {
+  return prefill_shape_ok(T, Hq, Hkv, max_len) &&
+         balanced_grid(T, Hq, Hkv, max_len, kv8 != 0,
+                       ws != 0 && prefill_wide_ws_bytes(T, Hq, Hkv, max_len) > 0) > 0;
 }
 
 extern "C" hipError_t qe_attn_prefill_ws(const void* q, const void* kc, const void* vc,

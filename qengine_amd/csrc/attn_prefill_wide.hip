@@ -82,12 +82,13 @@ __device__ __forceinline__ int tiles_of(const Call& s, int pos0, int u) {
   return max(1, (attended(s, pos0, u) + BN - 1) / BN);
 }
 
+constexpr float ROUND = 13.f;  // steps of a round of units outside the tile loop
 // Estimated time, in tile steps, of the last r units (n tiles each) cut into S slices.
 __host__ __device__ inline float slice_cost(int r, int W, int Hkv, int S, float n) {
   const int items = r * S;
   if (S > 1 && items > 2 * W) return 1e30f;
   const float rounds = items <= W ? 1.f : items <= 2 * W ? 2.f : 3.f;
-  return rounds * (n / (float)S + 13.f) + (S > 1 ? 6.f + 0.025f * (float)(items * Hkv) : 0.f);
+  return rounds * (n / (float)S + ROUND) + (S > 1 ? 6.f + 0.025f * (float)(items * Hkv) : 0.f);
 }
 // Slices of the cache that the last r units are cut into: the count with the least estimated time.
 __device__ __forceinline__ int slices(const Call& s, int pos0, int lane) {
@@ -683,18 +684,37 @@ static wide::Call plan(int T, int Hq, int Hkv, int max_len) {
   s.grp_m = magic(s.grp), s.Hkv_m = magic(Hkv), s.r_m = magic(s.r ? s.r : 1);
   return s;
 }
-// Slices for the longest prefix the cache can hold: 1 if no position can make cutting pay.
-static int most_slices(const wide::Call& s) {
-  const float n = (float)((s.max_len + tile::BN - 1) / tile::BN);
+// Slices of the last r units at n tiles each (the kernels' slices()).
+static int fewest_steps(const wide::Call& s, float n) {
   int best = 1;
   for (int S = 2; s.r && S <= WAVE; ++S)
     if (wide::slice_cost(s.r, s.W, s.Hkv, S, n) < wide::slice_cost(s.r, s.W, s.Hkv, best, n)) best = S;
   return best;
 }
+// ... for the longest prefix the cache can hold: 1 if no position can make cutting pay.
+static int most_slices(const wide::Call& s) {
+  return fewest_steps(s, (float)((s.max_len + tile::BN - 1) / tile::BN));
+}
 
 bool qe::prefill_wide_valid(int T, int Hq, int Hkv) {
   const wide::Call s = plan(T, Hq, Hkv, 1);
   return ((long)s.U + 2 * s.W) * Hkv <= 0x7fffffffL && (long)T * s.grp < 0x7fffffffL - wide::UCOLS;
+}
+
+// Whole rounds run their units' average length; the last r units are the shortest ones, alone on the
+// CUs (faster tiles) or in slices; no call ends before its longest unit.
+float qe::prefill_wide_steps(int T, int Hq, int Hkv, int max_len, bool kv8, bool ws) {
+  const wide::Call s = plan(T, Hq, Hkv, max_len);
+  const float pos = (float)(max_len > T ? max_len - T : 0), rows = (float)T, part = (float)s.r / (float)s.U;
+  float steps = (float)(s.U / s.W) * ((pos + rows * (1.f + part) / 2) / tile::BN + wide::ROUND);
+  if (s.r) {
+    const float n = (pos + rows * part) / tile::BN;
+    const int S = ws ? fewest_steps(s, n) : 1;
+    steps += S > 1 ? wide::slice_cost(s.r, s.W, s.Hkv, S, n) + (kv8 ? 12.f : 0.f)
+                   : (n + wide::ROUND) * (0.8f + 0.2f * (float)s.r / (float)s.W);
+  }
+  const float longest = (pos + rows) / tile::BN + wide::ROUND;
+  return steps > longest ? steps : longest;
 }
 
 size_t qe::prefill_wide_ws_bytes(int T, int Hq, int Hkv, int max_len) {

@@ -604,3 +604,36 @@ def test_capi_prefill_workspace_size(capi):
     assert size(40, 24, 4, 128) == 0
     assert size(2048, 24, 4, 4096) == 0   # 256 balanced workgroups
     assert size(2049, 24, 4, 4096) == slots
+
+
+# (rows, Hq, Hkv, position, fp8 cache, workspace) and us per call on 256 compute units, balanced and 32
+# columns per wave (in slices where there is a workspace)
+PREFILL_TIMES = [
+    ((1500, 24, 4, 4000, 0, 0), 198.5, 233.4), ((1500, 24, 4, 4000, 0, 1), 198.5, 179.8),
+    ((1500, 24, 4, 16000, 1, 0), 692.4, 960.0), ((1500, 24, 4, 16000, 1, 1), 692.4, 636.9),
+    ((777, 24, 4, 4000, 0, 0), 170.3, 119.7), ((1280, 24, 4, 16000, 1, 0), 673.4, 537.0),
+    ((2048, 24, 4, 4000, 0, 1), 240.9, 247.3), ((2048, 24, 4, 4000, 1, 1), 251.5, 274.4),
+    ((2049, 24, 4, 4000, 0, 0), 403.0, 268.4), ((3000, 24, 4, 16000, 1, 0), 1489.1, 1548.6),
+    ((3000, 24, 4, 16000, 1, 1), 1489.1, 1268.0), ((4096, 24, 4, 16000, 1, 1), 1628.8, 1716.9),
+    ((4096, 24, 4, 0, 1, 1), 253.4, 241.8), ((6144, 24, 4, 16000, 0, 0), 2517.8, 2592.4),
+    ((6144, 24, 4, 16000, 1, 1), 2644.5, 2804.9), ((8192, 24, 4, 16000, 0, 1), 3549.7, 3474.2),
+    ((8192, 24, 4, 16000, 1, 1), 3758.1, 3879.2), ((8192, 6, 1, 0, 1, 0), 234.4, 249.7),
+    ((4096, 6, 1, 16000, 0, 1), 624.6, 476.9), ((850, 48, 8, 16000, 0, 0), 695.3, 821.1),
+    ((1500, 48, 8, 0, 0, 0), 113.9, 85.3), ((3400, 12, 2, 16000, 1, 0), 752.1, 998.0),
+]
+
+
+@pytest.mark.parametrize("call,balanced,wide", PREFILL_TIMES)
+def test_prefill_dispatch_takes_the_faster_kernel(capi, call, balanced, wide):
+    """GQA 6 chunks run on the kernel that is faster at the end of their cache, with and without a
+    workspace."""
+    T, hq, hkv, pos, kv8, ws = call
+    f = capi.load().qe_attn_prefill_balanced
+    assert f(T, hq, hkv, pos + T, kv8, ws) == (balanced < wide)
+
+
+def test_prefill_dispatch_other_shapes(capi):
+    f = capi.load().qe_attn_prefill_balanced
+    assert f(2048, 32, 8, 4096, 0, 0) == 0  # another group size
+    assert f(2048, 25, 4, 4096, 0, 0) == 0 and f(0, 24, 4, 4096, 0, 0) == 0  # not a call
+    assert f(2048, 24, 4, 4096, 0, 1) == 1 and f(2048, 24, 4, 4096, 0, 0) == 1
