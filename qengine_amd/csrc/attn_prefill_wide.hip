@@ -511,7 +511,7 @@ attn_prefill_wide_kernel(const __bf16* __restrict__ q, const void* __restrict__ 
       run_tiles<KV8, decltype(mk)::value, decltype(sp)::value>(j0, j1, rg, cv, base, Lcol, lane, qb,
                                                                s.scale_log2, kop, sc, st);
     };
-    if (min(pos0 + r0 / SPLIT_ROWS * SPLIT_ROWS + 1, s.max_len) < SPLIT_BELOW) {
+    if (min(pos0 + (r0 & -SPLIT_ROWS) + 1, s.max_len) < SPLIT_BELOW) {
       run(K_{}, V_{}, J0, jm);
       run(V_{}, V_{}, jm, je);
     } else {
