@@ -112,10 +112,14 @@ hipError_t qe_attn_prefill(const void* q, const void* kc, const void* vc, const 
                            int max_len, float scale, hipStream_t stream);
 
 /* qe_attn_prefill with a caller's workspace, which lets a chunk that does not fill the CUs split
- * the cache over more of them: ws of at least qe_attn_prefill_ws_size() bytes, 16-byte aligned,
- * contents undefined before and after; calls that may overlap need one each. The size is 0 where no
- * position in the cache would make splitting pay. A null ws, or fewer bytes, runs unsplit (as
- * qe_attn_prefill does): the same values up to rounding. */
+ * the cache over more of them: ws of at least qe_attn_prefill_ws_need() bytes (kv8: on an fp8 cache),
+ * 16-byte aligned, contents undefined before and after; calls that may overlap need one each. The need
+ * is 0 where no position in the cache would make splitting pay. A null ws, or fewer bytes, runs unsplit
+ * (as qe_attn_prefill does): the same values up to rounding (the order of fp32 sums, and the running
+ * maximum against which the softmax weights are rounded to bf16). qe_attn_prefill_ws_size() is a bound
+ * of the need that holds for any T, max_len and cache type of Hkv heads, 0 where the need on a bf16
+ * cache is. */
+size_t qe_attn_prefill_ws_need(int T, int Hq, int Hkv, int max_len, int kv8);
 size_t qe_attn_prefill_ws_size(int T, int Hq, int Hkv, int max_len);
 hipError_t qe_attn_prefill_ws(const void* q, const void* kc, const void* vc, const int* pos,
                               const void* qg, long ldp, void* out, long ldo, int T, int Hq, int Hkv,

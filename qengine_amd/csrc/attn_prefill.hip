@@ -439,9 +439,13 @@ static hipError_t launch_prefill(const void* q, const void* kc, const void* vc, 
                              kv8, v_scale, w, stream);
 }
 
+extern "C" size_t qe_attn_prefill_ws_need(int T, int Hq, int Hkv, int max_len, int kv8) {
+  if (!prefill_shape_ok(T, Hq, Hkv, max_len)) return 0;
+  const size_t bytes = prefill_wide_ws_bytes(T, Hq, Hkv, max_len);
+  return bytes > 0 && balanced_grid(T, Hq, Hkv, max_len, kv8 != 0, true) ? 0 : bytes;
+}
 extern "C" size_t qe_attn_prefill_ws_size(int T, int Hq, int Hkv, int max_len) {
-  if (!prefill_shape_ok(T, Hq, Hkv, max_len) || balanced_grid(T, Hq, Hkv, max_len, false, true)) return 0;
-  return prefill_wide_ws_bytes(T, Hq, Hkv, max_len);
+  return qe_attn_prefill_ws_need(T, Hq, Hkv, max_len, 0) ? prefill_wide_ws_most(Hkv) : 0;
 }
 
 extern "C" int qe_attn_prefill_balanced(int T, int Hq, int Hkv, int max_len, int kv8, int ws) {

@@ -70,6 +70,7 @@ struct Call {
   int U;         // units of a KV head: 128 columns, column = row * grp + q head of the group
   int W;         // workgroups of a KV head that run at once
   int r;         // U % W: the units left when the others fill whole rounds
+  int most;      // slices that one of them is cut into at most
   uint32_t grp_m, r_m, Hkv_m;  // for udiv
   float scale_log2, v_scale;
   uint32_t q_flip;
@@ -92,7 +93,8 @@ __host__ __device__ inline float slice_cost(int r, int W, int Hkv, int S, float 
 }
 // Slices of the cache that the last r units are cut into: the count with the least estimated time.
 __device__ __forceinline__ int slices(const Call& s, int pos0, int lane) {
-  const float cost = slice_cost(s.r, s.W, s.Hkv, lane + 1, (float)tiles_of(s, pos0, s.r - 1));
+  const float n = (float)tiles_of(s, pos0, s.r - 1);
+  const float cost = lane < s.most ? slice_cost(s.r, s.W, s.Hkv, lane + 1, n) : 2e30f;
   float m = fminf(cost, dpp<0xB1>(cost));
   m = fminf(m, dpp<0x4E>(m));
   m = fminf(m, dpp<0x1B>(dpp<0x141>(m)));
@@ -541,7 +543,7 @@ attn_prefill_wide_kernel(const __bf16* __restrict__ q, const void* __restrict__ 
   const float L = xor32_pair(st.l, true);
   if (S > 1) {
     if (!wlive) return;
-    float* slot = ws + ((size_t)g * 2 * s.W + u * S + k) * SLOT_F;
+    float* slot = ws + ((size_t)g * s.r * s.most + u * S + k) * SLOT_F;
     f32x4_t* po = reinterpret_cast<f32x4_t*>(slot) + w * 32 * WAVE + lane;
 #pragma unroll
     for (int i = 0; i < 8; ++i)
@@ -614,7 +616,7 @@ attn_prefill_wide_combine(const int* __restrict__ pos_ptr, const __bf16* __restr
   if (r0 >= s.T) return;
   const int lc = c0 - r0 * s.grp + c, dr = udiv(lc, s.grp, s.grp_m);
   const int row = r0 + dr, hd = g * s.grp + lc - dr * s.grp;
-  const float* slots = ws + ((size_t)g * 2 * s.W + u * S) * SLOT_F;
+  const float* slots = ws + ((size_t)g * s.r * s.most + u * S) * SLOT_F;
   const float* ml = slots + UCOLS * HD + (w * WAVE + lane) * 2;
   const f32x4_t* po = reinterpret_cast<const f32x4_t*>(slots) + (w * 32 + ib * 2) * WAVE + lane;
   const int d0 = 16 * ib + 8 * h;
@@ -675,15 +677,6 @@ using namespace qe;
 // floor(2^32 / d) for udiv
 static uint32_t magic(int d) { return d == 1 ? 0xffffffffu : (uint32_t)((1ull << 32) / d); }
 
-static wide::Call plan(int T, int Hq, int Hkv, int max_len) {
-  wide::Call s{};
-  s.T = T, s.Hq = Hq, s.Hkv = Hkv, s.grp = Hq / Hkv, s.max_len = max_len;
-  s.U = (int)(((long)T * s.grp + wide::UCOLS - 1) / wide::UCOLS);
-  s.W = compute_units() / Hkv > 0 ? compute_units() / Hkv : 1;
-  s.r = s.U % s.W;
-  s.grp_m = magic(s.grp), s.Hkv_m = magic(Hkv), s.r_m = magic(s.r ? s.r : 1);
-  return s;
-}
 // Slices of the last r units at n tiles each (the kernels' slices()).
 static int fewest_steps(const wide::Call& s, float n) {
   int best = 1;
@@ -691,9 +684,16 @@ static int fewest_steps(const wide::Call& s, float n) {
     if (wide::slice_cost(s.r, s.W, s.Hkv, S, n) < wide::slice_cost(s.r, s.W, s.Hkv, best, n)) best = S;
   return best;
 }
-// ... for the longest prefix the cache can hold: 1 if no position can make cutting pay.
-static int most_slices(const wide::Call& s) {
-  return fewest_steps(s, (float)((s.max_len + tile::BN - 1) / tile::BN));
+// (`most`: the slices at the longest prefix the cache can hold; a shorter one takes no more)
+static wide::Call plan(int T, int Hq, int Hkv, int max_len) {
+  wide::Call s{};
+  s.T = T, s.Hq = Hq, s.Hkv = Hkv, s.grp = Hq / Hkv, s.max_len = max_len;
+  s.U = (int)(((long)T * s.grp + wide::UCOLS - 1) / wide::UCOLS);
+  s.W = compute_units() / Hkv > 0 ? compute_units() / Hkv : 1;
+  s.r = s.U % s.W;
+  s.most = fewest_steps(s, (float)((max_len + tile::BN - 1) / tile::BN));
+  s.grp_m = magic(s.grp), s.Hkv_m = magic(Hkv), s.r_m = magic(s.r ? s.r : 1);
+  return s;
 }
 
 bool qe::prefill_wide_valid(int T, int Hq, int Hkv) {
@@ -719,7 +719,10 @@ float qe::prefill_wide_steps(int T, int Hq, int Hkv, int max_len, bool kv8, bool
 
 size_t qe::prefill_wide_ws_bytes(int T, int Hq, int Hkv, int max_len) {
   const wide::Call s = plan(T, Hq, Hkv, max_len);
-  return most_slices(s) > 1 ? (size_t)Hkv * 2 * s.W * wide::SLOT_F * sizeof(float) : 0;
+  return s.most > 1 ? (size_t)Hkv * s.r * s.most * wide::SLOT_F * sizeof(float) : 0;
+}
+size_t qe::prefill_wide_ws_most(int Hkv) {
+  return (size_t)Hkv * 2 * plan(1, Hkv, Hkv, 1).W * wide::SLOT_F * sizeof(float);
 }
 
 hipError_t qe::launch_prefill_wide(const void* q, const void* kc, const void* vc, const int* pos,
@@ -733,8 +736,7 @@ hipError_t qe::launch_prefill_wide(const void* q, const void* kc, const void* vc
   s.scale_log2 = sl == 0.f ? 1.17549435e-38f : sl < 0.f ? -sl : sl;
   s.q_flip = sl < 0.f ? 0x80008000u : 0u;
   s.v_scale = v_scale, s.ldp = ldp, s.ldo = ldo;
-  const int most = s.r ? (2 * s.W / s.r < WAVE ? 2 * s.W / s.r : WAVE) : 1;  // slices per unit
-  const dim3 grid((unsigned)(s.U - s.r + s.r * (ws ? most : 1)) * Hkv), block(wide::WAVES * WAVE);
+  const dim3 grid((unsigned)(s.U - s.r + s.r * (ws ? s.most : 1)) * Hkv), block(wide::WAVES * WAVE);
   const auto* Q = static_cast<const __bf16*>(q);
   const auto* QG = static_cast<const __bf16*>(qg);
   auto* O = static_cast<__bf16*>(out);

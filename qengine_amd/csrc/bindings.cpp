@@ -235,8 +235,8 @@ struct RelaxedCaptureMode {
 // Workspace of a prefill call from torch's allocator (its block is reused in stream order), or an
 // undefined tensor: where the call needs none, where memory is short, and under stream capture, since
 // a capture that is not torch's own would keep the address of a block that goes back to the pool.
-torch::Tensor prefill_ws(const PrefillArgs& a, const torch::Tensor& like, hipStream_t stream) {
-  const size_t bytes = qe_attn_prefill_ws_size(a.T, a.Hq, a.Hkv, a.max_len);
+torch::Tensor prefill_ws(const PrefillArgs& a, bool kv8, const torch::Tensor& like, hipStream_t stream) {
+  const size_t bytes = qe_attn_prefill_ws_need(a.T, a.Hq, a.Hkv, a.max_len, kv8);
   hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
   if (bytes == 0 || hipStreamIsCapturing(stream, &st) != hipSuccess ||
       st != hipStreamCaptureStatusNone)
@@ -253,7 +253,7 @@ void attn_prefill(torch::Tensor q, torch::Tensor kc, torch::Tensor vc, torch::Te
                   torch::Tensor qg, torch::Tensor out) {
   const auto a = parse_prefill(q, kc, vc, pos, qg, out, true);
   const c10::DeviceGuard guard(q.device());
-  const auto ws = prefill_ws(a, q, stream_of(q));
+  const auto ws = prefill_ws(a, false, q, stream_of(q));
   raise_on(qe_attn_prefill_ws(q.data_ptr(), kc.data_ptr(), vc.data_ptr(), pos.data_ptr<int>(),
                               qg.data_ptr(), a.ldp, out.data_ptr(), a.ldo, a.T, a.Hq, a.Hkv,
                               a.max_len, 1.0f / 16.0f, ws.defined() ? ws.data_ptr() : nullptr,
@@ -377,7 +377,7 @@ void attn_prefill_fp8(torch::Tensor q, torch::Tensor kc8, torch::Tensor vc8, tor
   kv_scales(k_scale, v_scale);
   const auto a = parse_prefill(q, kc8, vc8, pos, qg, out, true, true);
   const c10::DeviceGuard guard(q.device());
-  const auto ws = prefill_ws(a, q, stream_of(q));
+  const auto ws = prefill_ws(a, true, q, stream_of(q));
   raise_on(qe_attn_prefill_fp8_ws(q.data_ptr(), kc8.data_ptr(), vc8.data_ptr(), pos.data_ptr<int>(),
                                   qg.data_ptr(), a.ldp, out.data_ptr(), a.ldo, a.T, a.Hq, a.Hkv,
                                   a.max_len, 1.0f / 16.0f, (float)k_scale, (float)v_scale,

@@ -637,3 +637,18 @@ def test_prefill_dispatch_other_shapes(capi):
     assert f(2048, 32, 8, 4096, 0, 0) == 0  # another group size
     assert f(2048, 25, 4, 4096, 0, 0) == 0 and f(0, 24, 4, 4096, 0, 0) == 0  # not a call
     assert f(2048, 24, 4, 4096, 0, 1) == 1 and f(2048, 24, 4, 4096, 0, 0) == 1
+
+
+def test_capi_prefill_workspace_need(capi):
+    """qe_attn_prefill_ws_need on 256 compute units: the slots that the call's last units can be cut into
+    and no more, never above qe_attn_prefill_ws_size, 0 where the call takes the balanced kernel."""
+    need, size = capi.prefill_ws_need, capi.load().qe_attn_prefill_ws_size
+    slot = (128 * D + 2 * 256) * 4
+    assert need(9, 16, 2, 32768) == 2 * 64 * slot         # one unit a KV head, at most 64 slices
+    assert need(301, 24, 4, 16384) == 4 * 15 * 4 * slot   # 15 units on 64 workgroups
+    assert need(1800, 24, 4, 5800) > 0 and need(1800, 24, 4, 5800, True) == 0
+    assert need(40, 24, 4, 128) == 0 and need(0, 24, 4, 4096) == 0 and need(16, 25, 4, 4096) == 0
+    for T in (1, 9, 64, 301, 777, 1400, 2049, 3000, 9001):
+        for hq, hkv in ((24, 4), (16, 2), (32, 8), (4, 4), (6, 1), (8, 8), (64, 1)):
+            for max_len in (64, 1000, 5000, 40000, 130000):
+                assert need(T, hq, hkv, max_len) <= size(T, hq, hkv, max_len)

@@ -4,7 +4,7 @@ import threading
 import pytest
 import torch
 
-from attn_cases import BF, D
+from attn_cases import BF, D, attn_close
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
@@ -60,3 +60,64 @@ def test_allocates_beside_another_threads_capture(native):
         torch.cuda.synchronize()
         assert (x == 2 * n).all()
     assert torch.equal(out, ref)
+
+
+SHAPES = [
+    # (Hq, Hkv, T, pos, max_len)
+    (16, 2, 9, 12000, 12100),    # one unit a KV head in many slices
+    (24, 4, 301, 5000, 5400),    # 15 units, 4 slices each
+    (32, 8, 600, 3000, 3600),    # whole rounds of units ahead of a remainder in slices (256 CUs)
+    (24, 4, 1400, 2000, 3400),   # the same, GQA 6
+    (24, 4, 40, 100, 9000),      # short prefix in a long cache: fewer slices than the workspace holds
+    (8, 2, 40, 5000, 3000),      # rows past the end of the cache
+]
+
+
+@pytest.mark.parametrize("kv8", [False, True])
+@pytest.mark.parametrize("hq,hkv,T,pos,max_len", SHAPES)
+def test_caller_workspace(native, capi, hq, hkv, T, pos, max_len, kv8):
+    """The C entry points on a workspace of exactly qe_attn_prefill_ws_need() bytes, full of NaN and
+    between guards: the op's bits, guards untouched. One byte less runs unsplit (the bits of the entry
+    point without a workspace); a misaligned one is rejected."""
+    q, kc, vc, p, qg, out = case(hq, hkv, T, pos, max_len)
+    need = capi.prefill_ws_need(T, hq, hkv, max_len, kv8)
+    assert need > 0 and need % 16 == 0
+    if kv8:
+        kc, vc = kc.to(torch.float8_e4m3fn), vc.to(torch.float8_e4m3fn)
+    scales = (0.5, 2.0) if kv8 else ()
+    guard = 4096
+    buf = torch.full((guard + need + guard,), 0xFF, dtype=torch.uint8, device=DEV)  # fp32 NaN
+    ws = buf.data_ptr() + guard
+    args = (q, kc, vc, p, qg, qg.stride(0))
+    rest = (hq * D, T, hq, hkv, max_len)
+    run_ws = capi.prefill_fp8_ws if kv8 else capi.prefill_ws
+    plain = capi.prefill_fp8 if kv8 else capi.prefill
+    op = native.attn_prefill_fp8 if kv8 else native.attn_prefill
+    ref, unsplit = torch.empty_like(out), torch.empty_like(out)
+    op(q, kc, vc, p, qg, ref, *scales)
+    assert plain(*args, unsplit, *rest, *scales) == 0
+    assert run_ws(*args, out, *rest, *scales, ws, need) == 0
+    torch.cuda.synchronize()
+    assert torch.isfinite(out.float()).all() and torch.equal(out, ref)
+    assert (buf[:guard] == 0xFF).all() and (buf[guard + need:] == 0xFF).all()
+    assert run_ws(*args, out.fill_(float("nan")), *rest, *scales, ws, need - 1) == 0
+    assert torch.equal(out, unsplit)
+    assert run_ws(*args, out.fill_(float("nan")), *rest, *scales, None, 0) == 0
+    assert torch.equal(out, unsplit)
+    assert run_ws(*args, out, *rest, *scales, ws + 8, need) == capi.HIP_ERROR_INVALID_VALUE
+    ok, mx, mean = attn_close(ref.cpu(), unsplit.cpu())
+    assert ok, (mx, mean)
+
+
+def test_op_allocates_what_it_needs(native, capi):
+    """An eager chunk takes the bytes that its slices need from torch's allocator, and holds none of
+    them once it has returned."""
+    *args, out = case(16, 2, 9, 8000)
+    native.attn_prefill(*args, out)
+    torch.cuda.synchronize()
+    before = torch.cuda.memory_allocated()
+    torch.cuda.reset_peak_memory_stats()
+    native.attn_prefill(*args, out)
+    need = capi.prefill_ws_need(9, 16, 2, 8009)
+    assert need <= torch.cuda.max_memory_allocated() - before <= need + (2 << 20)
+    assert torch.cuda.memory_allocated() == before
