@@ -30,6 +30,7 @@ from ._C import (  # noqa: E402,F401
     attn_decode_fp8_partials,
     attn_decode_partials,
     attn_prefill,
+    attn_prefill_ws,
     attn_prep,
     attn_prep_chunk,
     attn_prep_decode,
@@ -40,6 +41,7 @@ from ._C import (  # noqa: E402,F401
     gemv_bf16,
     l2_persist_limit,
     mtp_select,
+    prefill_ws_bytes,
     rmsnorm1p,
     set_gdn_early,
     set_gdn_phases,
@@ -85,3 +87,11 @@ def alloc_partials(n_rows: int, hq: int, ns: int, device="cuda"):
     po = torch.empty(n_rows, hq, ns, HEAD_DIM, dtype=torch.float32, device=device)
     pml = torch.empty(n_rows, hq, ns, 2, dtype=torch.float32, device=device)
     return po, pml
+
+
+def alloc_prefill_ws(rows: int, hq: int, hkv: int, max_len: int, kv8: bool = False, device="cuda"):
+    """Caller-owned workspace of ``attn_prefill_ws`` / ``attn_prefill_fp8_ws`` for chunks of ``rows``
+    rows (another row count may need more: take the largest). With it a call allocates nothing, and
+    a captured call splits the cache as an eager one does, with the same bits."""
+    n = prefill_ws_bytes(rows, hq, hkv, max_len, kv8)
+    return torch.empty(n, dtype=torch.uint8, device=device)

@@ -1,8 +1,10 @@
 // torch bindings for qengine_amd._C: the reference's qengine._C attention ops with the same
 // Python signatures and the same validation contract (reference csrc/bindings.cpp:1-30,147-183).
 // Every op writes into caller-provided tensors, enqueues on the current HIP stream and never syncs,
-// so it can be captured in a hipGraph. None allocates, except the prefill ops outside a capture
-// (prefill_ws). Row-batched arguments are 2-D views
+// so it can be captured in a hipGraph. None allocates, except attn_prefill and attn_prefill_fp8
+// outside a capture, which take a workspace from torch's allocator (prefill_ws; an allocator short of
+// memory gives its cached blocks back first, which can wait for the device). Row-batched arguments
+// are 2-D views
 // [n, width] with stride(1) == 1 and any row stride (a 1-D tensor counts as one row).
 //
 // Each op is a thin shell over the C ABI in include/qe_attn.h. Launch errors are raised as
@@ -249,16 +251,37 @@ torch::Tensor prefill_ws(const PrefillArgs& a, bool kv8, const torch::Tensor& li
   }
 }
 
-void attn_prefill(torch::Tensor q, torch::Tensor kc, torch::Tensor vc, torch::Tensor pos,
-                  torch::Tensor qg, torch::Tensor out) {
-  const auto a = parse_prefill(q, kc, vc, pos, qg, out, true);
-  const c10::DeviceGuard guard(q.device());
-  const auto ws = prefill_ws(a, false, q, stream_of(q));
+// A caller's workspace of a prefill call: an empty one runs unsplit.
+void chk_ws(const torch::Tensor& ws, const torch::Tensor& q) {
+  TORCH_CHECK(ws.device() == q.device() && ws.is_contiguous(), "ws must be contiguous, on q's device");
+  TORCH_CHECK(reinterpret_cast<uintptr_t>(ws.data_ptr()) % 16 == 0, "ws must be 16-byte aligned");
+}
+
+void launch_prefill(const torch::Tensor& q, const torch::Tensor& kc, const torch::Tensor& vc,
+                    const torch::Tensor& pos, const torch::Tensor& qg, const torch::Tensor& out,
+                    const PrefillArgs& a, const torch::Tensor& ws) {
   raise_on(qe_attn_prefill_ws(q.data_ptr(), kc.data_ptr(), vc.data_ptr(), pos.data_ptr<int>(),
                               qg.data_ptr(), a.ldp, out.data_ptr(), a.ldo, a.T, a.Hq, a.Hkv,
                               a.max_len, 1.0f / 16.0f, ws.defined() ? ws.data_ptr() : nullptr,
                               ws.defined() ? ws.nbytes() : 0, stream_of(q)),
            "qe_attn_prefill");
+}
+
+void attn_prefill(torch::Tensor q, torch::Tensor kc, torch::Tensor vc, torch::Tensor pos,
+                  torch::Tensor qg, torch::Tensor out) {
+  const auto a = parse_prefill(q, kc, vc, pos, qg, out, true);
+  const c10::DeviceGuard guard(q.device());
+  launch_prefill(q, kc, vc, pos, qg, out, a, prefill_ws(a, false, q, stream_of(q)));
+}
+
+// attn_prefill on a caller's workspace: it allocates nothing, and a captured call has the eager
+// call's bits.
+void attn_prefill_ws(torch::Tensor q, torch::Tensor kc, torch::Tensor vc, torch::Tensor pos,
+                     torch::Tensor qg, torch::Tensor out, torch::Tensor ws) {
+  const auto a = parse_prefill(q, kc, vc, pos, qg, out, true);
+  chk_ws(ws, q);
+  const c10::DeviceGuard guard(q.device());
+  launch_prefill(q, kc, vc, pos, qg, out, a, ws);
 }
 
 // q: [n, Hq*256] contiguous; part_o: fp32 [>=n, Hq, NS, 256]; part_ml: [>=n, Hq, NS, 2];
@@ -372,18 +395,33 @@ void attn_prep_fp8(torch::Tensor qg, torch::Tensor k, torch::Tensor v, torch::Te
 }
 
 // attn_prefill over the fp8 cache (kc8/vc8 [Hkv, max_len, 256] E4M3FN codes).
-void attn_prefill_fp8(torch::Tensor q, torch::Tensor kc8, torch::Tensor vc8, torch::Tensor pos,
-                      torch::Tensor qg, torch::Tensor out, double k_scale, double v_scale) {
-  kv_scales(k_scale, v_scale);
-  const auto a = parse_prefill(q, kc8, vc8, pos, qg, out, true, true);
-  const c10::DeviceGuard guard(q.device());
-  const auto ws = prefill_ws(a, true, q, stream_of(q));
+void launch_prefill_fp8(const torch::Tensor& q, const torch::Tensor& kc8, const torch::Tensor& vc8,
+                        const torch::Tensor& pos, const torch::Tensor& qg, const torch::Tensor& out,
+                        const PrefillArgs& a, double k_scale, double v_scale, const torch::Tensor& ws) {
   raise_on(qe_attn_prefill_fp8_ws(q.data_ptr(), kc8.data_ptr(), vc8.data_ptr(), pos.data_ptr<int>(),
                                   qg.data_ptr(), a.ldp, out.data_ptr(), a.ldo, a.T, a.Hq, a.Hkv,
                                   a.max_len, 1.0f / 16.0f, (float)k_scale, (float)v_scale,
                                   ws.defined() ? ws.data_ptr() : nullptr,
                                   ws.defined() ? ws.nbytes() : 0, stream_of(q)),
            "qe_attn_prefill_fp8");
+}
+
+void attn_prefill_fp8(torch::Tensor q, torch::Tensor kc8, torch::Tensor vc8, torch::Tensor pos,
+                      torch::Tensor qg, torch::Tensor out, double k_scale, double v_scale) {
+  kv_scales(k_scale, v_scale);
+  const auto a = parse_prefill(q, kc8, vc8, pos, qg, out, true, true);
+  const c10::DeviceGuard guard(q.device());
+  launch_prefill_fp8(q, kc8, vc8, pos, qg, out, a, k_scale, v_scale, prefill_ws(a, true, q, stream_of(q)));
+}
+
+void attn_prefill_fp8_ws(torch::Tensor q, torch::Tensor kc8, torch::Tensor vc8, torch::Tensor pos,
+                         torch::Tensor qg, torch::Tensor out, double k_scale, double v_scale,
+                         torch::Tensor ws) {
+  kv_scales(k_scale, v_scale);
+  const auto a = parse_prefill(q, kc8, vc8, pos, qg, out, true, true);
+  chk_ws(ws, q);
+  const c10::DeviceGuard guard(q.device());
+  launch_prefill_fp8(q, kc8, vc8, pos, qg, out, a, k_scale, v_scale, ws);
 }
 
 void attn_decode_fp8(torch::Tensor q, torch::Tensor kc8, torch::Tensor vc8, torch::Tensor pos,
@@ -693,6 +731,13 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("attn_prep_chunk", &attn_prep_chunk, "attn_prep without the 8-row limit (prefill chunks)");
   m.def("attn_prefill", &attn_prefill,
         "chunked-prefill gated attention over the KV cache (q, kc, vc, pos, qg, out)");
+  m.def("attn_prefill_ws", &attn_prefill_ws,
+        "attn_prefill on a caller's workspace (q, kc, vc, pos, qg, out, ws)");
+  m.def("prefill_ws_bytes",
+        [](int T, int Hq, int Hkv, int max_len, bool kv8) {
+          return (int64_t)qe_attn_prefill_ws_need(T, Hq, Hkv, max_len, kv8);
+        },
+        "bytes of the workspace that lets a prefill call split the cache (T, Hq, Hkv, max_len, kv8)");
   m.def("split_size", [](int max_len, int NS) { return qe_attn_split_size(max_len, NS); },
         "cache positions per split-KV slice for (max_len, NS)");
   m.def("version", []() { return std::string(qe_attn_version()); });
@@ -720,6 +765,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         "eps, k_scale, v_scale)");
   m.def("attn_prefill_fp8", &attn_prefill_fp8,
         "attn_prefill over the fp8 cache (q, kc8, vc8, pos, qg, out, k_scale, v_scale)");
+  m.def("attn_prefill_fp8_ws", &attn_prefill_fp8_ws,
+        "attn_prefill_fp8 on a caller's workspace (q, kc8, vc8, pos, qg, out, k_scale, v_scale, ws)");
   m.def("attn_decode_fp8", &attn_decode_fp8,
         "attn_decode over the fp8 KV cache (q, kc8, vc8, pos, qg, part_o, part_ml, out, k_scale, "
         "v_scale)");

@@ -121,3 +121,55 @@ def test_op_allocates_what_it_needs(native, capi):
     need = capi.prefill_ws_need(9, 16, 2, 8009)
     assert need <= torch.cuda.max_memory_allocated() - before <= need + (2 << 20)
     assert torch.cuda.memory_allocated() == before
+
+
+@pytest.mark.parametrize("kv8", [False, True])
+def test_captured_on_a_caller_workspace_equals_eager(native, kv8):
+    """On a caller's workspace a captured chunk splits the cache as the eager op does: every replay, the
+    position changed in place and eager calls between them, has the eager op's bits. The call allocates
+    nothing."""
+    import qengine_amd as qa
+    hq, hkv, T, max_len = 24, 4, 60, 4096
+    q, kc, vc, p, qg, out = case(hq, hkv, T, 3000, max_len)
+    if kv8:
+        kc, vc = kc.to(torch.float8_e4m3fn), vc.to(torch.float8_e4m3fn)
+    scales = (0.5, 2.0) if kv8 else ()
+    op = native.attn_prefill_fp8 if kv8 else native.attn_prefill
+    op_ws = native.attn_prefill_fp8_ws if kv8 else native.attn_prefill_ws
+    ws = qa.alloc_prefill_ws(T, hq, hkv, max_len, kv8)
+    assert ws.numel() > 0
+    eager = torch.empty_like(out)
+    op_ws(q, kc, vc, p, qg, out, *scales, ws)
+    torch.cuda.synchronize()
+    torch.cuda.reset_peak_memory_stats()
+    before = torch.cuda.memory_allocated()
+    op_ws(q, kc, vc, p, qg, out, *scales, ws)
+    assert torch.cuda.max_memory_allocated() == before
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        op_ws(q, kc, vc, p, qg, out, *scales, ws)
+    for pos in (3000, 0, 4000, 1234):
+        p.fill_(pos)
+        out.fill_(float("nan"))
+        ws.fill_(0xFF)
+        graph.replay()
+        op(q, kc, vc, p, qg, eager, *scales)
+        torch.cuda.synchronize()
+        assert torch.equal(out, eager), pos
+
+
+def test_workspace_op_rejects(native):
+    """A workspace that is misaligned, strided or elsewhere is refused; an empty one runs unsplit."""
+    q, kc, vc, p, qg, out = case(24, 4, 60, 3000)
+    ws = torch.empty(1 << 26, dtype=torch.uint8, device=DEV)
+    for bad, why in ((ws[8:], "aligned"), (ws[::2], "contiguous"), (ws.cpu(), "device")):
+        with pytest.raises(RuntimeError, match=why):
+            native.attn_prefill_ws(q, kc, vc, p, qg, out, bad)
+    native.attn_prefill_ws(q, kc, vc, p, qg, out, ws[:0])
+    ref = torch.empty_like(out)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):  # attn_prefill takes no workspace under capture
+        native.attn_prefill(q, kc, vc, p, qg, ref)
+    graph.replay()
+    torch.cuda.synchronize()
+    assert torch.equal(out, ref)
