@@ -193,3 +193,14 @@ def test_rows_of_two_term_blocks(native, hq, hkv):
             same.append(out.view(T, hq, D)[r, h] == (p @ V[h // grp, :L]).to(BF))
     share = torch.stack(same).float().mean(1).view(len(rows), hq).mean(1)
     assert share.min() > 0.99, share
+
+
+@pytest.mark.parametrize("hq,hkv,T,pos", [(4, 2, 70, 0), (4, 2, 129, 40), (2, 2, 33, 0), (10, 2, 27, 5),
+                                          (14, 2, 19, 0)])
+def test_group_sizes(native, hq, hkv, T, pos):
+    """Rows and heads of a lane's columns for group sizes that divide, straddle and exceed its step of two
+    columns, with rows that end inside a wave."""
+    q, kc, vc, qg = inputs(hq, hkv, T, pos + T, 6)
+    out = run(native.attn_prefill, q, kc, vc, pos, qg)
+    ok, mx, mean = attn_close(out, O.attn_prefill(q, kc, vc, pos, qg, hq))
+    assert ok, (mx, mean)
