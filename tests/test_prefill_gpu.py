@@ -31,11 +31,11 @@ def run_prefill(C, q, kc, vc, pos, qg):
     (24, 4, 128, 1000, 1100),  # cache longer than the chunk needs
     (4, 4, 64, 0, 64),         # no GQA
     (24, 4, 200, 100, 250),    # rows past the end of the cache attend the whole cache
-    (12, 2, 16, 0, 16),        # GQA 6, one 16-row block (the balanced layout's half pair)
-    (24, 4, 17, 3, 30),        # GQA 6, two blocks, the second ragged
-    (6, 1, 48, 700, 760),      # GQA 6, one KV head, three blocks
-    (24, 4, 150, 30, 180),     # GQA 6, 10 blocks: an odd number (5) of workgroups per KV head
-    (6, 1, 80, 0, 80),         # GQA 6, 5 blocks (3 workgroups, the last block's quad part-empty)
+    (12, 2, 16, 0, 16),        # GQA 6, 16 rows
+    (24, 4, 17, 3, 30),        # GQA 6, 17 rows
+    (6, 1, 48, 700, 760),      # GQA 6, one KV head
+    (24, 4, 150, 30, 180),     # GQA 6, rows straddle the waves of 32 columns
+    (6, 1, 80, 0, 80),         # GQA 6, from an empty cache
 ])
 def test_prefill_matches_oracle(native, hq, hkv, T, pos, max_len):
     g = gen(hq * 1000 + T)
@@ -48,7 +48,7 @@ def test_prefill_matches_oracle(native, hq, hkv, T, pos, max_len):
     assert ok, (mx, mean)
 
 
-@pytest.mark.parametrize("hq,hkv", [(8, 2), (24, 4)])  # the 8-wave and the balanced layout
+@pytest.mark.parametrize("hq,hkv", [(8, 2), (24, 4)])
 def test_prefill_ignores_unattended_cache(native, hq, hkv):
     T, pos, max_len = 96, 40, 400
     g = gen(77 + hq)

@@ -66,7 +66,7 @@ SHAPES = [
     # (Hq, Hkv, T, pos, max_len)
     (16, 2, 9, 12000, 12100),    # one unit a KV head in many slices
     (24, 4, 301, 5000, 5400),    # 15 units, 4 slices each
-    (32, 8, 600, 3000, 3600),    # whole rounds of units ahead of a remainder in slices (256 CUs)
+    (32, 8, 1100, 3000, 4100),   # a whole round of units ahead of a remainder in slices (256 CUs)
     (24, 4, 1400, 2000, 3400),   # the same, GQA 6
     (24, 4, 40, 100, 9000),      # short prefix in a long cache: fewer slices than the workspace holds
     (8, 2, 40, 5000, 3000),      # rows past the end of the cache
