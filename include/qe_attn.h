@@ -112,23 +112,22 @@ hipError_t qe_attn_prefill(const void* q, const void* kc, const void* vc, const 
                            int max_len, float scale, hipStream_t stream);
 
 /* qe_attn_prefill with a caller's workspace, which lets a chunk that does not fill the CUs split
- * the cache over more of them: ws of at least qe_attn_prefill_ws_need() bytes (kv8: on an fp8 cache),
- * 16-byte aligned, contents undefined before and after; calls that may overlap need one each. The need
+ * the cache over more of them: ws of at least qe_attn_prefill_ws_need() bytes, 16-byte
+ * aligned, contents undefined before and after; calls that may overlap need one each. The need
  * is 0 where no position in the cache would make splitting pay. A null ws, or fewer bytes, runs unsplit
  * (as qe_attn_prefill does): the same values up to rounding (the order of fp32 sums, and the running
  * maximum against which the softmax weights are rounded to bf16). qe_attn_prefill_ws_size() is a bound
- * of the need that holds for any T, max_len and cache type of Hkv heads, 0 where the need on a bf16
- * cache is. */
-size_t qe_attn_prefill_ws_need(int T, int Hq, int Hkv, int max_len, int kv8);
+ * of the need that holds for any T and max_len of Hkv heads, 0 where the need is. */
+size_t qe_attn_prefill_ws_need(int T, int Hq, int Hkv, int max_len);
 size_t qe_attn_prefill_ws_size(int T, int Hq, int Hkv, int max_len);
 hipError_t qe_attn_prefill_ws(const void* q, const void* kc, const void* vc, const int* pos,
                               const void* qg, long ldp, void* out, long ldo, int T, int Hq, int Hkv,
                               int max_len, float scale, void* ws, size_t ws_bytes,
                               hipStream_t stream);
 
-/* 1 where such a prefill call (kv8: on an fp8 cache; ws: with a workspace of the size above) runs the
+/* 1 where such a prefill call (ws: with a workspace of the size above), on either cache, runs the
  * kernel that pairs long and short row blocks, 0 where it runs the one of 32 columns per wave. */
-int qe_attn_prefill_balanced(int T, int Hq, int Hkv, int max_len, int kv8, int ws);
+int qe_attn_prefill_balanced(int T, int Hq, int Hkv, int max_len, int ws);
 
 /* Number of cache positions per split-KV slice for a row attending L positions with NS partial
  * slots: ceil(L/NS) rounded up to a multiple of 32 (at least 32); row t's partial s covers

@@ -89,9 +89,9 @@ def alloc_partials(n_rows: int, hq: int, ns: int, device="cuda"):
     return po, pml
 
 
-def alloc_prefill_ws(rows: int, hq: int, hkv: int, max_len: int, kv8: bool = False, device="cuda"):
+def alloc_prefill_ws(rows: int, hq: int, hkv: int, max_len: int, device="cuda"):
     """Caller-owned workspace of ``attn_prefill_ws`` / ``attn_prefill_fp8_ws`` for chunks of ``rows``
     rows (another row count may need more: take the largest). With it a call allocates nothing, and
     a captured call splits the cache as an eager one does, with the same bits."""
-    n = prefill_ws_bytes(rows, hq, hkv, max_len, kv8)
+    n = prefill_ws_bytes(rows, hq, hkv, max_len)
     return torch.empty(n, dtype=torch.uint8, device=device)

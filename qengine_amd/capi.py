@@ -32,8 +32,8 @@ SIGNATURES = {
     "qe_attn_prefill_fp8_ws": (_I, [_P, _P, _P, _P, _P, _L, _P, _L, _I, _I, _I, _I, _F, _F, _F, _P,
                                     _Z, _P]),
     "qe_attn_prefill_ws_size": (_Z, [_I, _I, _I, _I]),
-    "qe_attn_prefill_ws_need": (_Z, [_I, _I, _I, _I, _I]),
-    "qe_attn_prefill_balanced": (_I, [_I, _I, _I, _I, _I, _I]),
+    "qe_attn_prefill_ws_need": (_Z, [_I, _I, _I, _I]),
+    "qe_attn_prefill_balanced": (_I, [_I, _I, _I, _I, _I]),
     "qe_attn_prefill_fp8": (_I, [_P, _P, _P, _P, _P, _L, _P, _L, _I, _I, _I, _I, _F, _F, _F, _P]),
     "qe_attn_prep_decode": (_I, [_P, _P, _P, _L, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _L, _I, _I,
                                  _I, _I, _I, _I, _F, _F, _P]),
@@ -158,9 +158,9 @@ def prefill_fp8(q, kc8, vc8, pos, qg, ldp, out, ldo, T, hq, hkv, max_len, k_scal
                                       _stream(stream))
 
 
-def prefill_ws_need(T, hq, hkv, max_len, kv8=False) -> int:
+def prefill_ws_need(T, hq, hkv, max_len) -> int:
     """Bytes of the workspace that lets such a call split the cache (qe_attn_prefill_ws_need)."""
-    return load().qe_attn_prefill_ws_need(T, hq, hkv, max_len, int(kv8))
+    return load().qe_attn_prefill_ws_need(T, hq, hkv, max_len)
 
 
 def prefill_ws(q, kc, vc, pos, qg, ldp, out, ldo, T, hq, hkv, max_len, ws, ws_bytes, scale=1.0 / 16,

@@ -379,24 +379,26 @@ using namespace qe;
 // The balanced kernel's grid if it takes the call, else 0: GQA 6 where its estimated time is less than
 // the wide kernel's (prefill_wide_steps, in whose unit it is), at the last chunk that fits the cache:
 // the position is known to the device alone, and a wide call's lead is largest on a short prefix, so
-// a call that runs wide is the faster one wherever it stands. A round of 256 workgroups takes 1.48 (bf16
-// cache) or 1.37 (fp8) steps for a tile of the prefix plus 0.6 of the chunk, and 35 or 30 outside the
-// tile loop; a part-empty last round nearly as much. Against both kernels timed at 24 / 4, 6 / 1, 12 / 2 and
-// 48 / 8 heads, 256 to 16,384 rows on 0 to 16,000 positions, both caches, with and without slices, the
-// choice at the call's own position costs 0.1% on average and 6% at most (1,960 rows of an empty fp8
-// cache). us per call, balanced / wide in slices / wide unsliced, 24 / 4 heads:
+// a call that runs wide is the faster one wherever it stands. A round of 256 workgroups takes 1.4 steps for
+// a tile of the prefix plus 0.6 of the chunk, and 31 outside the tile loop; a part-empty last round nearly
+// as much. One rule for both caches, so that an fp8 cache with scales of 1 has the bits of the bf16 cache:
+// measured alone they fit 1.48 and 35 (bf16), 1.37 and 30 (fp8). Against both kernels timed at 24 / 4,
+// 6 / 1, 12 / 2 and 48 / 8 heads, 256 to 16,384 rows on 0 to 16,000 positions, with and without slices, the
+// choice costs 0.4% (bf16) and 0.1% (fp8) on average; where it runs wide the balanced kernel is at most 4%
+// faster (3,000 rows on 16,000 fp8 positions unsliced), where it runs balanced the wide one at most 10% (1,960
+// rows of an empty bf16 cache). us per call, balanced / wide in slices / wide unsliced, 24 / 4 heads:
 //   bf16, 2,048 rows on 4,000: 241 / 247 / 264, 1,500 on 4,000 198 / 180 / 233, 4,096 on 16,000 1,584 / - / 1,564
 //   fp8, 2,048 rows on 4,000: 252 / 274 / 305, 1,500 on 4,000 221 / 203 / 270, 4,096 on 16,000 1,629 / - / 1,717
-static int balanced_grid(int T, int Hq, int Hkv, int max_len, bool kv8, bool ws) {
+static int balanced_grid(int T, int Hq, int Hkv, int max_len, bool ws) {
   if (Hq != prefill::BAL_GRP * Hkv) return 0;
   const long wgs = ((T + 15) / 16 + 1) / 2 * (long)Hkv;
   if (wgs > 0x7fffffffL) return 0;
   const int cus = compute_units();
   const float pos = (float)(max_len > T ? max_len - T : 0);
-  const float round = (kv8 ? 1.37f : 1.48f) * (pos + 0.6f * (float)T) / tile::BN + (kv8 ? 30.f : 35.f);
+  const float round = 1.4f * (pos + 0.6f * (float)T) / tile::BN + 31.f;
   const float part = (float)(wgs % cus) / (float)cus;
   const float steps = round * ((float)(wgs / cus) + (part > 0.f ? 0.9f + 0.1f * part : 0.f));
-  return steps < prefill_wide_steps(T, Hq, Hkv, max_len, kv8, ws) ? (int)wgs : 0;
+  return steps < prefill_wide_steps(T, Hq, Hkv, max_len, ws) ? (int)wgs : 0;
 }
 
 static bool prefill_shape_ok(int T, int Hq, int Hkv, int max_len) {
@@ -417,7 +419,7 @@ static hipError_t launch_prefill(const void* q, const void* kc, const void* vc, 
     return hipErrorInvalidValue;
   const size_t need = prefill_wide_ws_bytes(T, Hq, Hkv, max_len);
   float* w = ws && need && ws_bytes >= need ? static_cast<float*>(ws) : nullptr;
-  if (const int grid = balanced_grid(T, Hq, Hkv, max_len, kv8, w != nullptr)) {
+  if (const int grid = balanced_grid(T, Hq, Hkv, max_len, w != nullptr)) {
     // KV-head-per-XCD placement when the heads divide the XCDs evenly and every XCD of a head gets
     // the same number of workgroups
     const int per_head = prefill::XCDS % Hkv == 0 ? prefill::XCDS / Hkv : 0;
@@ -439,19 +441,18 @@ static hipError_t launch_prefill(const void* q, const void* kc, const void* vc, 
                              kv8, v_scale, w, stream);
 }
 
-extern "C" size_t qe_attn_prefill_ws_need(int T, int Hq, int Hkv, int max_len, int kv8) {
+extern "C" size_t qe_attn_prefill_ws_need(int T, int Hq, int Hkv, int max_len) {
   if (!prefill_shape_ok(T, Hq, Hkv, max_len)) return 0;
   const size_t bytes = prefill_wide_ws_bytes(T, Hq, Hkv, max_len);
-  return bytes > 0 && balanced_grid(T, Hq, Hkv, max_len, kv8 != 0, true) ? 0 : bytes;
+  return bytes > 0 && balanced_grid(T, Hq, Hkv, max_len, true) ? 0 : bytes;
 }
 extern "C" size_t qe_attn_prefill_ws_size(int T, int Hq, int Hkv, int max_len) {
-  return qe_attn_prefill_ws_need(T, Hq, Hkv, max_len, 0) ? prefill_wide_ws_most(Hkv) : 0;
+  return qe_attn_prefill_ws_need(T, Hq, Hkv, max_len) ? prefill_wide_ws_most(Hkv) : 0;
 }
 
-extern "C" int qe_attn_prefill_balanced(int T, int Hq, int Hkv, int max_len, int kv8, int ws) {
+extern "C" int qe_attn_prefill_balanced(int T, int Hq, int Hkv, int max_len, int ws) {
   return prefill_shape_ok(T, Hq, Hkv, max_len) &&
-         balanced_grid(T, Hq, Hkv, max_len, kv8 != 0,
-                       ws != 0 && prefill_wide_ws_bytes(T, Hq, Hkv, max_len) > 0) > 0;
+         balanced_grid(T, Hq, Hkv, max_len, ws != 0 && prefill_wide_ws_bytes(T, Hq, Hkv, max_len) > 0) > 0;
 }
 
 extern "C" hipError_t qe_attn_prefill_ws(const void* q, const void* kc, const void* vc,

@@ -9,7 +9,7 @@ namespace qe {
 bool prefill_wide_valid(int T, int Hq, int Hkv);
 // Estimated time of a call whose chunk ends the cache, in steps: the time of one tile of 32 positions
 // in a full round of units (0.9 us on the bf16 cache, 1.0 us on the fp8 cache). ws: with a workspace.
-float prefill_wide_steps(int T, int Hq, int Hkv, int max_len, bool kv8, bool ws);
+float prefill_wide_steps(int T, int Hq, int Hkv, int max_len, bool ws);
 // Workspace with which a call cuts units into slices; 0 where it never would. At most
 // prefill_wide_ws_most(): two slots for every workgroup that runs at once.
 size_t prefill_wide_ws_bytes(int T, int Hq, int Hkv, int max_len);

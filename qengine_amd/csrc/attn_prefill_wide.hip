@@ -735,15 +735,16 @@ bool qe::prefill_wide_valid(int T, int Hq, int Hkv) {
 }
 
 // Whole rounds run their units' average length; the last r units are the shortest ones, alone on the
-// CUs (faster tiles) or in slices; no call ends before its longest unit.
-float qe::prefill_wide_steps(int T, int Hq, int Hkv, int max_len, bool kv8, bool ws) {
+// CUs (faster tiles) or in slices (9 steps are the fp8 cache's first tiles, converted per slice); no call
+// ends before its longest unit.
+float qe::prefill_wide_steps(int T, int Hq, int Hkv, int max_len, bool ws) {
   const wide::Call s = plan(T, Hq, Hkv, max_len);
   const float pos = (float)(max_len > T ? max_len - T : 0), rows = (float)T, part = (float)s.r / (float)s.U;
   float steps = (float)(s.U / s.W) * ((pos + rows * (1.f + part) / 2) / tile::BN + wide::ROUND);
   if (s.r) {
     const float n = (pos + rows * part) / tile::BN;
     const int S = ws ? fewest_steps(s, n) : 1;
-    steps += S > 1 ? wide::slice_cost(s.r, s.W, s.Hkv, S, n) + (kv8 ? 12.f : 0.f)
+    steps += S > 1 ? wide::slice_cost(s.r, s.W, s.Hkv, S, n) + 9.f
                    : (n + wide::ROUND) * (0.8f + 0.2f * (float)s.r / (float)s.W);
   }
   const float longest = (pos + rows) / tile::BN + wide::ROUND;

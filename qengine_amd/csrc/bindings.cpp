@@ -237,8 +237,8 @@ struct RelaxedCaptureMode {
 // Workspace of a prefill call from torch's allocator (its block is reused in stream order), or an
 // undefined tensor: where the call needs none, where memory is short, and under stream capture, since
 // a capture that is not torch's own would keep the address of a block that goes back to the pool.
-torch::Tensor prefill_ws(const PrefillArgs& a, bool kv8, const torch::Tensor& like, hipStream_t stream) {
-  const size_t bytes = qe_attn_prefill_ws_need(a.T, a.Hq, a.Hkv, a.max_len, kv8);
+torch::Tensor prefill_ws(const PrefillArgs& a, const torch::Tensor& like, hipStream_t stream) {
+  const size_t bytes = qe_attn_prefill_ws_need(a.T, a.Hq, a.Hkv, a.max_len);
   hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
   if (bytes == 0 || hipStreamIsCapturing(stream, &st) != hipSuccess ||
       st != hipStreamCaptureStatusNone)
@@ -271,7 +271,7 @@ void attn_prefill(torch::Tensor q, torch::Tensor kc, torch::Tensor vc, torch::Te
                   torch::Tensor qg, torch::Tensor out) {
   const auto a = parse_prefill(q, kc, vc, pos, qg, out, true);
   const c10::DeviceGuard guard(q.device());
-  launch_prefill(q, kc, vc, pos, qg, out, a, prefill_ws(a, false, q, stream_of(q)));
+  launch_prefill(q, kc, vc, pos, qg, out, a, prefill_ws(a, q, stream_of(q)));
 }
 
 // attn_prefill on a caller's workspace: it allocates nothing, and a captured call has the eager
@@ -411,7 +411,7 @@ void attn_prefill_fp8(torch::Tensor q, torch::Tensor kc8, torch::Tensor vc8, tor
   kv_scales(k_scale, v_scale);
   const auto a = parse_prefill(q, kc8, vc8, pos, qg, out, true, true);
   const c10::DeviceGuard guard(q.device());
-  launch_prefill_fp8(q, kc8, vc8, pos, qg, out, a, k_scale, v_scale, prefill_ws(a, true, q, stream_of(q)));
+  launch_prefill_fp8(q, kc8, vc8, pos, qg, out, a, k_scale, v_scale, prefill_ws(a, q, stream_of(q)));
 }
 
 void attn_prefill_fp8_ws(torch::Tensor q, torch::Tensor kc8, torch::Tensor vc8, torch::Tensor pos,
@@ -734,10 +734,10 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("attn_prefill_ws", &attn_prefill_ws,
         "attn_prefill on a caller's workspace (q, kc, vc, pos, qg, out, ws)");
   m.def("prefill_ws_bytes",
-        [](int T, int Hq, int Hkv, int max_len, bool kv8) {
-          return (int64_t)qe_attn_prefill_ws_need(T, Hq, Hkv, max_len, kv8);
+        [](int T, int Hq, int Hkv, int max_len) {
+          return (int64_t)qe_attn_prefill_ws_need(T, Hq, Hkv, max_len);
         },
-        "bytes of the workspace that lets a prefill call split the cache (T, Hq, Hkv, max_len, kv8)");
+        "bytes of the workspace that lets a prefill call split the cache (T, Hq, Hkv, max_len)");
   m.def("split_size", [](int max_len, int NS) { return qe_attn_split_size(max_len, NS); },
         "cache positions per split-KV slice for (max_len, NS)");
   m.def("version", []() { return std::string(qe_attn_version()); });

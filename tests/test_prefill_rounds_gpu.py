@@ -78,6 +78,7 @@ BALANCED = [
     (12, 2, 3500, 0, 9000),
     (48, 8, 900, 100, 9000),    # one XCD per KV head
     (6, 1, 8000, 0, 9000),
+    (24, 4, 4096, 0, 20096),    # two rounds; alone, the bf16 cache's fastest kernel is the other one
     (24, 4, 6144, 0, 22144),    # three rounds
 ]
 
@@ -86,7 +87,7 @@ BALANCED = [
 @pytest.mark.parametrize("hq,hkv,T,pos,max_len", BALANCED)
 def test_balanced(native, capi, hq, hkv, T, pos, max_len, kv8):
     if qa.compute_units() == 256:
-        assert capi.load().qe_attn_prefill_balanced(T, hq, hkv, max_len, int(kv8), 0)
+        assert capi.load().qe_attn_prefill_balanced(T, hq, hkv, max_len, 0)
     scales = (2.0, 0.5) if kv8 else (1.0, 1.0)
     q, kc, vc, p, qg = make(hq, hkv, T, pos, max_len, kv8)
     check(call(capi, q, kc, vc, p, qg, scales=scales), exact(q, kc, vc, pos, qg, *scales))
@@ -102,7 +103,7 @@ def test_balanced_two_term_rows(native, capi, kv8):
     value is the exact attention's bf16 rounding (one term: about 3 in 5)."""
     hq, hkv, T, pos, max_len = 24, 4, 1999, 7, 6000
     if qa.compute_units() == 256:
-        assert capi.load().qe_attn_prefill_balanced(T, hq, hkv, max_len, int(kv8), 0)
+        assert capi.load().qe_attn_prefill_balanced(T, hq, hkv, max_len, 0)
     q, kc, vc, p, qg = make(hq, hkv, T, pos, max_len, kv8, seed=3)
     qg.fill_(60.0)
     out, ref = call(capi, q, kc, vc, p, qg), exact(q, kc, vc, pos, qg)
@@ -128,12 +129,12 @@ def test_rounds_of_units(native, capi, hq, hkv, T, pos, kv8):
     if qa.compute_units() == 256:
         U, W = -(-T * (hq // hkv) // 128), 256 // hkv
         assert U >= W or T == 40
-        need = capi.prefill_ws_need(T, hq, hkv, max_len, kv8)
+        need = capi.prefill_ws_need(T, hq, hkv, max_len)
         assert (need > 0) == (U % W != 0)
-        assert not capi.load().qe_attn_prefill_balanced(T, hq, hkv, max_len, int(kv8), 1)
+        assert not capi.load().qe_attn_prefill_balanced(T, hq, hkv, max_len, 1)
     scales = (2.0, 0.5) if kv8 else (1.0, 1.0)
     q, kc, vc, p, qg = make(hq, hkv, T, pos, max_len, kv8)
     ref = exact(q, kc, vc, pos, qg, *scales)
-    ws = qa.alloc_prefill_ws(T, hq, hkv, max_len, kv8).fill_(0xFF)
+    ws = qa.alloc_prefill_ws(T, hq, hkv, max_len).fill_(0xFF)
     check(call(capi, q, kc, vc, p, qg, ws, scales), ref)
     check(call(capi, q, kc, vc, p, qg, scales=scales), ref)

@@ -80,7 +80,7 @@ def test_caller_workspace(native, capi, hq, hkv, T, pos, max_len, kv8):
     between guards: the op's bits, guards untouched. One byte less runs unsplit (the bits of the entry
     point without a workspace); a misaligned one is rejected."""
     q, kc, vc, p, qg, out = case(hq, hkv, T, pos, max_len)
-    need = capi.prefill_ws_need(T, hq, hkv, max_len, kv8)
+    need = capi.prefill_ws_need(T, hq, hkv, max_len)
     assert need > 0 and need % 16 == 0
     if kv8:
         kc, vc = kc.to(torch.float8_e4m3fn), vc.to(torch.float8_e4m3fn)
@@ -136,7 +136,7 @@ def test_captured_on_a_caller_workspace_equals_eager(native, kv8):
     scales = (0.5, 2.0) if kv8 else ()
     op = native.attn_prefill_fp8 if kv8 else native.attn_prefill
     op_ws = native.attn_prefill_fp8_ws if kv8 else native.attn_prefill_ws
-    ws = qa.alloc_prefill_ws(T, hq, hkv, max_len, kv8)
+    ws = qa.alloc_prefill_ws(T, hq, hkv, max_len)
     assert ws.numel() > 0
     eager = torch.empty_like(out)
     op_ws(q, kc, vc, p, qg, out, *scales, ws)
