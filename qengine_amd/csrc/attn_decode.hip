@@ -1001,24 +1001,22 @@ constexpr int TILE_U4 = TILE * ROW_CHUNKS;   // 16-byte slots of one K (or V) ti
 constexpr int REGION_U4 = 2 * TILE_U4;       // a subset's K tile then V tile
 }  // namespace cols
 
-// Look-ahead rounds of attn_partials_cols_kernel (one column tile per wave). bf16 cache: round
-// 0's K and V tiles load together; after that the V tile of round r loads while the subset
-// computes S^T and the softmax of round r, and the K tile of round r+1 while it computes
-// O^T += V^T P^T. fp8 cache: the fp8 K tile of round r+1 loads into the subset's 8 KB staging
-// buffer during S^T and the softmax of round r, is converted into the bf16 K tile, and the fp8
-// V tile of round r+1 then loads into the same buffer during O^T += V^T P^T. Each half takes its
-// LDS operands and the LDS-DMA target as distinct __restrict__ pointers, so the compiler's
-// wait-count pass sees that the operand reads do not depend on the DMA just issued (without that
-// it waits for it before the first read).
+// Look-ahead rounds of attn_partials_cols_kernel. bf16 cache: round 0's K and V tiles load together;
+// after that the V tile of round r loads while the subset computes S^T and the softmax of round r, and
+// the K tile of round r+1 while it computes O^T += V^T P^T. fp8 cache, one column tile per wave: the fp8
+// K tile of round r+1 loads into the subset's 8 KB staging buffer during S^T and the softmax of round r,
+// is converted into the bf16 K tile, and the fp8 V tile of round r+1 then loads into the same buffer
+// during O^T += V^T P^T. No operand read may wait for the loads just issued: on the fp8 cache each half
+// takes its LDS operands and the LDS-DMA target as distinct __restrict__ pointers, on the bf16 cache the
+// target is a plain LDS address (otherwise the compiler's wait-count pass waits for the loads before the
+// first read).
 namespace cols {
 constexpr int STAGE8_U4 = TILE * HD / 16;  // 16-byte slots of one fp8 tile: 8 KB
-// Operand reads kept ahead of the MFMAs in S^T and O^T (tile::qk_tile / pv_tile_tr LEAD) at one
-// column tile per wave. Same-box harness A/B, partials us, none -> 4: 5 rows at 4101 (config 3)
-// 10.64 -> 10.42, 8 rows at 4104 13.45 -> 13.39, 8 rows at 16392 22.80 -> 22.49; bits identical.
-// Two column tiles per wave already spill and keep the compiler's order.
-template <int CPW>
-constexpr int LEAD = CPW == 1 ? 4 : 0;
-constexpr int PLEAD = 4;  // qk_pairs and pv_pairs: operand reads in flight
+// Operand reads kept ahead of the MFMAs in S^T and O^T. Same-box harness A/B at one column tile per wave,
+// partials us, none -> 4: 5 rows at 4101 (config 3) 10.64 -> 10.42, 8 rows at 4104 13.45 -> 13.39, 8 rows
+// at 16392 22.80 -> 22.49; bits identical. Two column tiles per wave on the fp8 cache spill and keep
+// the compiler's order.
+constexpr int LEAD = 4;
 
 // 8 one-KB LDS-DMA loads of an fp8 tile, rows 4i .. 4i+3, row-major (chunk q of row r at 16 r + q)
 __device__ __forceinline__ void issue_fp8(__amdgpu_buffer_rsrc_t rs, int p0, u32x4_t* dst, int rank,
@@ -1067,7 +1065,7 @@ __device__ __forceinline__ void qk_pairs(const char* __restrict__ kt, const bf16
   };
   bf16x8_t op[16];
 #pragma unroll
-  for (int k = 0; k < PLEAD; ++k) op[k] = read(k);
+  for (int k = 0; k < LEAD; ++k) op[k] = read(k);
 #pragma unroll
   for (int u = 0; u < CPW; ++u) sacc[u][0] = sacc[u][1] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   __builtin_amdgcn_sched_barrier(0);
@@ -1075,7 +1073,7 @@ __device__ __forceinline__ void qk_pairs(const char* __restrict__ kt, const bf16
   for (int k = 0; k < 16; ++k) {
 #pragma unroll
     for (int u = 0; u < CPW; ++u) sacc[u][k >> 3] = mfma16x16x32(op[k], qb[u][k & 7], sacc[u][k >> 3]);
-    if (k + PLEAD < 16) op[k + PLEAD] = read(k + PLEAD);
+    if (k + LEAD < 16) op[k + LEAD] = read(k + LEAD);
     __builtin_amdgcn_sched_barrier(0);
   }
 }
@@ -1098,7 +1096,7 @@ __device__ __forceinline__ void pv_pairs(const char* __restrict__ vt, int lane,
   };
   bf16x8_t op[16];
 #pragma unroll
-  for (int i = 0; i < PLEAD; ++i) op[i] = read(i);
+  for (int i = 0; i < LEAD; ++i) op[i] = read(i);
   __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
   for (int i = 0; i < 16; ++i) {
@@ -1107,7 +1105,7 @@ __device__ __forceinline__ void pv_pairs(const char* __restrict__ vt, int lane,
       acc[u][i] = mfma16x16x32(op[i], as_bf16x8(hi[u]), acc[u][i]);
       acc[u][i] = mfma16x16x32(op[i], as_bf16x8(lo[u]), acc[u][i]);
     }
-    if (i + PLEAD < 16) op[i + PLEAD] = read(i + PLEAD);
+    if (i + LEAD < 16) op[i + LEAD] = read(i + LEAD);
     __builtin_amdgcn_sched_barrier(0);
   }
 }
@@ -1152,7 +1150,7 @@ __device__ __forceinline__ void qk_softmax_half(
   if (load) issue_fp8(rs, p_load, dst, rank, wps, lane);
   if (!has) return;
   f32x4_t sacc[CPW][2];
-  tile::qk_tile<CPW, false, LEAD<CPW>>(kt, qb, c, g4, sacc);
+  tile::qk_tile<CPW, false, LEAD>(kt, qb, c, g4, sacc);
   softmax<CPW>(sacc, p0, Lmin, Lcol, scale_log2, g4, m, l, acc, pb_hi, pb_lo);
 }
 template <int CPW>
@@ -1163,7 +1161,7 @@ __device__ __forceinline__ void pv_half_la(const u32x4_t* __restrict__ vt,
                                            const u32x4_t (&pb_hi)[CPW], const u32x4_t (&pb_lo)[CPW],
                                            f32x4_t (&acc)[CPW][16]) {
   if (load) issue_fp8(rs, p_load, dst, rank, wps, lane);
-  if (has) tile::pv_tile_tr<CPW, true, false, LEAD<CPW>>(vt, lane, g4, pb_hi, pb_lo, acc);
+  if (has) tile::pv_tile_tr<CPW, true, false, LEAD>(vt, lane, g4, pb_hi, pb_lo, acc);
 }
 // All NTH threads of the workgroup convert the fp8 tiles of the first nact subsets once, from
 // `src` (row-major) to `dst` (the bf16 K or V tile layout) in each subset's region of `region`
@@ -1284,11 +1282,11 @@ attn_partials_cols_kernel(const __bf16* __restrict__ q, const __bf16* __restrict
         Lcol[u] = in_pass((rank * CPW + u) * 16 + cc, grp, P)
                       ? min(pos0 + ((rank * CPW + u) * 16 + cc) / grp + 1, max_len) : 0;
     };
-    const uint32_t bytes = (uint32_t)P.end * (uint32_t)(HD * ELEM);
-    const __amdgpu_buffer_rsrc_t krs =
-        make_rsrc_uniform(reinterpret_cast<const char*>(kc) + head_off, bytes);
-    const __amdgpu_buffer_rsrc_t vrs =
-        make_rsrc_uniform(reinterpret_cast<const char*>(vc) + head_off, bytes);
+    // fp8 cache: the KV head's rows up to the pass's end
+    const auto head_rsrc = [&](const __bf16* base) __attribute__((always_inline)) {
+      return make_rsrc_uniform(reinterpret_cast<const char*>(base) + head_off,
+                               (uint32_t)P.end * (uint32_t)(HD * ELEM));
+    };
 
     float m[CPW], l[CPW];
     f32x4_t acc[CPW][16];  // tile::pv_tile_tr layout
@@ -1334,6 +1332,7 @@ attn_partials_cols_kernel(const __bf16* __restrict__ q, const __bf16* __restrict
         __syncthreads();  // K of round r+1 has landed; V of round r is no longer read
       }
     } else if constexpr (LA8) {
+      const __amdgpu_buffer_rsrc_t krs = head_rsrc(kc), vrs = head_rsrc(vc);
       constexpr int NTH = SUB * WPS * WAVE;
       const auto nact = [&](int r) {  // active subsets of round r (>= 1 for r < rounds)
         return min(SUB, (P.end - (P.beg + r * SUB * TILE) + TILE - 1) / TILE);
@@ -1378,23 +1377,23 @@ attn_partials_cols_kernel(const __bf16* __restrict__ q, const __bf16* __restrict
           __syncthreads();  // bf16 V of round r+1 whole; the staging buffer is free
         }
       }
-    } else
-    for (int r = 0; r < rounds; ++r) {
-      if (r == 0) lcol();
-      const int p0 = P.beg + (r * SUB + sub) * TILE;  // this subset's tile in round r
-      const bool has = p0 < P.end;                     // uniform per subset
-      if (has) {
-        // fp8: 8 loads of K then 8 of V, one KB (rows 4j .. 4j+3) each, shared by the subset's
-        // waves: 16-byte chunk q of row r of K at vt[16 r + q], of V at vt[512 + 16 r + q].
-        for (int i = rank; i < 16; i += WPS) {
-          const int row = 4 * (i & 7) + (lane >> 4);
-          buffer_load16_to_lds(i < 8 ? krs : vrs, (uint32_t)(p0 + row) * HD + (lane & 15) * 16,
-                               vt + 64 * i);
+    } else {  // fp8 cache, two column tiles per wave: no look-ahead (no registers for it)
+      const __amdgpu_buffer_rsrc_t krs = head_rsrc(kc), vrs = head_rsrc(vc);
+      for (int r = 0; r < rounds; ++r) {
+        if (r == 0) lcol();
+        const int p0 = P.beg + (r * SUB + sub) * TILE;  // this subset's tile in round r
+        const bool has = p0 < P.end;                     // uniform per subset
+        if (has) {
+          // fp8: 8 loads of K then 8 of V, one KB (rows 4j .. 4j+3) each, shared by the subset's
+          // waves: 16-byte chunk q of row r of K at vt[16 r + q], of V at vt[512 + 16 r + q].
+          for (int i = rank; i < 16; i += WPS) {
+            const int row = 4 * (i & 7) + (lane >> 4);
+            buffer_load16_to_lds(i < 8 ? krs : vrs, (uint32_t)(p0 + row) * HD + (lane & 15) * 16,
+                                 vt + 64 * i);
+          }
         }
-      }
-      vmcnt_wait<0>();
-      __syncthreads();  // every wave's loads of this round have landed
-      if constexpr (KV8) {
+        vmcnt_wait<0>();
+        __syncthreads();  // every wave's loads of this round have landed
         // Convert once, all waves of the workgroup together: chunk gk of the active subsets'
         // tiles (subset gk / 512, chunk gk % 512) goes to thread gk % (64 SUB WPS).
         constexpr int CHUNKS = TILE * HD / 16;  // 16-byte fp8 chunks per tile
@@ -1432,19 +1431,19 @@ attn_partials_cols_kernel(const __bf16* __restrict__ q, const __bf16* __restrict
           }
         }
         __builtin_amdgcn_sched_barrier(0);  // keep the K operand reads below the conversion
+        f32x4_t sacc[CPW][2];
+        u32x4_t pb_hi[CPW], pb_lo[CPW];
+        if (has) {
+          tile::qk_tile<CPW, false, 0>(kt, qb, c, g4, sacc);
+          if (p0 + TILE > P.Lmin)
+            tile::softmax_tile<CPW, true, true>(sacc, p0, Lcol, scale_log2, g4, m, l, acc, pb_hi, pb_lo);
+          else
+            tile::softmax_tile<CPW, false, true>(sacc, p0, Lcol, scale_log2, g4, m, l, acc, pb_hi, pb_lo);
+        }
+        __syncthreads();  // the bf16 V tile is whole
+        if (has) tile::pv_tile_tr<CPW, true, false, 0>(vt, lane, g4, pb_hi, pb_lo, acc);
+        __syncthreads();  // this round's tiles are read before the next round overwrites them
       }
-      f32x4_t sacc[CPW][2];
-      u32x4_t pb_hi[CPW], pb_lo[CPW];
-      if (has) {
-        tile::qk_tile<CPW, false, cols::LEAD<CPW>>(kt, qb, c, g4, sacc);
-        if (p0 + TILE > P.Lmin)
-          tile::softmax_tile<CPW, true, true>(sacc, p0, Lcol, scale_log2, g4, m, l, acc, pb_hi, pb_lo);
-        else
-          tile::softmax_tile<CPW, false, true>(sacc, p0, Lcol, scale_log2, g4, m, l, acc, pb_hi, pb_lo);
-      }
-      if constexpr (KV8) __syncthreads();  // the bf16 V tile is whole
-      if (has) tile::pv_tile_tr<CPW, true, false, cols::LEAD<CPW>>(vt, lane, g4, pb_hi, pb_lo, acc);
-      __syncthreads();  // this round's tiles are read before the next round overwrites them
     }
 
     // ---- merge the 4 subsets in order 0..3 (as attn_partials_kernel merges its waves). Subsets
