@@ -8,17 +8,19 @@
 //  * One wave per SIMD, so the overlap is inside the wave: step j runs S^T of tile j + 1 beside the
 //    softmax of tile j, whose second half runs beside the first MFMAs of O^T of tile j. The order is
 //    pinned by a scheduling barrier after each MFMA. The loop is bound by the instructions a lone
-//    wave can issue (about 4 clocks each: 236 of them and 16 exponentials against 1,024 clocks of
-//    MFMA per tile): 1,540 clocks a tile on a 12k cache; 2,110 with S^T, softmax and O^T in turn.
+//    wave can issue: 205 of them a tile (VALU with 32 MFMAs and 16 exponentials, LDS, scalar) take about
+//    1,650 clocks against 1,024 of MFMA (counters, 12k caches; at 1.8 to 1.9 GHz under this load).
 //  * K and V arrive by LDS DMA in a ring of four stages, one instruction between two MFMAs (issued
 //    together they held the wave up: 0.16 us of the 0.98 us a tile then took).
 //  * Where the units do not fill the CUs (short chunks on long caches above all), the last U mod W
 //    units of a KV head are cut into slices of the cache (slices()); their partials go through a
 //    workspace and a second kernel merges them. The slice count depends on the attended length,
 //    which only the device knows, so both kernels compute it.
-// Measured against the kernels this one replaced, 24 / 4 heads, bf16 cache, us per call: 301 rows on
-// 12,007 positions 415 -> 100; 64 on 4,000 149 -> 25; 512 on 512 48 -> 30; 777 on none 41 -> 30;
-// 1,500 on 1,000 92 -> 80; 2,048 rows on 2,048 at 32 / 8 heads 229 -> 193 and at 16 / 2 138 -> 114.
+// Measured against the kernels this one replaced, 24 / 4 heads, bf16 cache, us per call (unsplit without a
+// workspace): 301 rows on 12,007 positions 420 -> 107 (unsplit 277); 64 on 4,000 151 -> 27 (99); 777 on
+// none 42 -> 30; 1,500 on 4,000 196 -> 182; 2,048 rows on 2,048 at 32 / 8 heads 233 -> 198 and at 16 / 2
+// 138 -> 114. One unit of an empty cache (9 to 32 rows at group sizes above 1) 11.3 .. 12.0 -> 12.0: the
+// epilogue of 32 columns is longer than that of 16.
 #include "attn_tile.hpp"
 #include "attn_prefill.hpp"
 
@@ -84,7 +86,13 @@ __device__ __forceinline__ int tiles_of(const Call& s, int pos0, int u) {
 }
 
 constexpr float ROUND = 13.f;  // steps of a round of units outside the tile loop
-// Estimated time, in tile steps, of the last r units (n tiles each) cut into S slices.
+// Estimated time, in tile steps (0.9 us in a full round, bf16 cache), of the last r units (n tiles each)
+// cut into S slices: rounds of r S workgroups, and for S > 1 the second kernel, 6 steps and 0.025 for each
+// of the slots it reads. Fitted to 24 / 4 heads; checked against 26 calls at 24 / 4, 16 / 2, 4 / 4, 32 / 8, 8 / 1
+// and 64 / 8 heads, both caches, 9 to 1,500 rows on 1,000 to 16,000 positions, each timed at up to 20 slice
+// counts: the count with the least estimate is within 2% of the fastest one in 13, within 8% in 21; it is
+// too large for one or a few units on short prefixes (24% at 100 rows on 2,000 at 4 / 4: 26 slices
+// 21.4 us, 12 17.2).
 __host__ __device__ inline float slice_cost(int r, int W, int Hkv, int S, float n) {
   const int items = r * S;
   if (S > 1 && items > 2 * W) return 1e30f;
