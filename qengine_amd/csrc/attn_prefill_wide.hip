@@ -721,24 +721,32 @@ static uint32_t magic(int d) { return d == 1 ? 0xffffffffu : (uint32_t)((1ull <<
 // Slices of the last r units at n tiles each (the kernels' slices()).
 static int fewest_steps(const wide::Call& s, float n) {
   int best = 1;
-  for (int S = 2; s.r && S <= WAVE; ++S)
-    if (wide::slice_cost(s.r, s.W, s.Hkv, S, n) < wide::slice_cost(s.r, s.W, s.Hkv, best, n)) best = S;
+  float least = wide::slice_cost(s.r, s.W, s.Hkv, 1, n);
+  for (int S = 2; s.r && S <= WAVE && s.r * S <= 2 * s.W; ++S) {
+    const float cost = wide::slice_cost(s.r, s.W, s.Hkv, S, n);
+    if (cost < least) least = cost, best = S;
+  }
   return best;
 }
-// (`most`: the slices at the longest prefix the cache can hold; a shorter one takes no more)
-static wide::Call plan(int T, int Hq, int Hkv, int max_len) {
+static wide::Call units(int T, int Hq, int Hkv) {
   wide::Call s{};
-  s.T = T, s.Hq = Hq, s.Hkv = Hkv, s.grp = Hq / Hkv, s.max_len = max_len;
+  s.T = T, s.Hq = Hq, s.Hkv = Hkv, s.grp = Hq / Hkv;
   s.U = (int)(((long)T * s.grp + wide::UCOLS - 1) / wide::UCOLS);
   s.W = compute_units() / Hkv > 0 ? compute_units() / Hkv : 1;
   s.r = s.U % s.W;
-  s.most = fewest_steps(s, (float)((max_len + tile::BN - 1) / tile::BN));
+  return s;
+}
+// (`most`: the slices at the longest prefix the cache can hold; a shorter one takes no more)
+static wide::Call plan(int T, int Hq, int Hkv, int max_len) {
+  wide::Call s = units(T, Hq, Hkv);
+  s.max_len = max_len;
+  s.most = fewest_steps(s, (float)(((long)max_len + tile::BN - 1) / tile::BN));
   s.grp_m = magic(s.grp), s.Hkv_m = magic(Hkv), s.r_m = magic(s.r ? s.r : 1);
   return s;
 }
 
 bool qe::prefill_wide_valid(int T, int Hq, int Hkv) {
-  const wide::Call s = plan(T, Hq, Hkv, 1);
+  const wide::Call s = units(T, Hq, Hkv);
   return ((long)s.U + 2 * s.W) * Hkv <= 0x7fffffffL && (long)T * s.grp < 0x7fffffffL - wide::UCOLS;
 }
 
@@ -746,7 +754,7 @@ bool qe::prefill_wide_valid(int T, int Hq, int Hkv) {
 // CUs (faster tiles) or in slices (9 steps are the fp8 cache's first tiles, converted per slice); no call
 // ends before its longest unit.
 float qe::prefill_wide_steps(int T, int Hq, int Hkv, int max_len, bool ws) {
-  const wide::Call s = plan(T, Hq, Hkv, max_len);
+  const wide::Call s = units(T, Hq, Hkv);
   const float pos = (float)(max_len > T ? max_len - T : 0), rows = (float)T, part = (float)s.r / (float)s.U;
   float steps = (float)(s.U / s.W) * ((pos + rows * (1.f + part) / 2) / tile::BN + wide::ROUND);
   if (s.r) {
@@ -764,7 +772,7 @@ size_t qe::prefill_wide_ws_bytes(int T, int Hq, int Hkv, int max_len) {
   return s.most > 1 ? (size_t)Hkv * s.r * s.most * wide::SLOT_F * sizeof(float) : 0;
 }
 size_t qe::prefill_wide_ws_most(int Hkv) {
-  return (size_t)Hkv * 2 * plan(1, Hkv, Hkv, 1).W * wide::SLOT_F * sizeof(float);
+  return (size_t)Hkv * 2 * units(1, Hkv, Hkv).W * wide::SLOT_F * sizeof(float);
 }
 
 hipError_t qe::launch_prefill_wide(const void* q, const void* kc, const void* vc, const int* pos,
